@@ -177,7 +177,7 @@ PROBES_BTD = ("btd_level", "btd_tail", "beam_assemble", "shell_assemble")
 PROBES_BAND = ("band_panel", "band_update", "band_sweep", "beam_assemble", "shell_assemble")
 PROBES_FRONTS = ("front_step", "front_assemble", "front_solve", "beam_assemble", "shell_assemble")
 
-KERNEL_NAMES = {"btd_level": "btd_level_kernel", "btd_tail": "btd_tail_kernel",
+KERNEL_NAMES = {"btd_level": "cr_reduce_kernel (per halving of the rows)", "btd_tail": "cr_reduce_kernel (last rows)",
                 "band_panel": "band_batch_inv_kernel", "band_update": "band_step_kernel",
                 "band_sweep": "band_batch_apply_kernel + band_couple_kernel",
                 "beam_assemble": "beam_assemble_kernel<0>", "shell_assemble": "shell_element_kernel",

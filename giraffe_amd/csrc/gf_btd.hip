@@ -1,5 +1,7 @@
-// Block-tridiagonal cyclic reduction on gfx950: the tangent solve for narrow
-// bands (replaces sparsesystem -> MKL PARDISO, src/SparseMatrix.cpp:74-166).
+// FP32 block-tridiagonal cyclic reduction on gfx950 with the factors kept: the
+// preconditioner of the mixed-precision refinement for narrow bands (replaces
+// sparsesystem -> MKL PARDISO, src/SparseMatrix.cpp:74-166).  The FP64 systems
+// are factored and solved in one pass by gf_cr.hip.
 //
 // A band matrix of half-bandwidth b, cut into diagonal blocks of size m >= b,
 // is block-tridiagonal: rows of block i couple only to blocks i-1 (A_i), i (B_i)
@@ -8,11 +10,10 @@
 //   eliminated row e:  Binv_e = B_e^-1,  X_e = Binv_e A_e,  Y_e = Binv_e C_e
 //   kept row k (neighbours l = p-1, r = p+1):
 //       B_k -= A_k Y_l + C_k X_r,   A_k <- -A_k X_l,   C_k <- -C_k Y_r
-// until one block row (the top) is left.  The right-hand side follows the same
-// levels (z_e = Binv_e f_e, f_k -= A_k z_l + C_k z_r with the pre-update A_k,
-// C_k) and back-substitution runs the levels in reverse
-// (x_e = z_e - X_e x_l - Y_e x_r).  Active row p at level L is global block
-// row (p+1)*2^L - 1.
+// until one block row (the top) is left.  A solve runs the right-hand side
+// through the levels (z_e = Binv_e f_e, f_k -= A_k z_l + C_k z_r with the
+// pre-update A_k, C_k), then back (x_e = z_e - X_e x_l - Y_e x_r).  Active row p
+// at level L is global block row (p+1)*2^L - 1.
 //
 // gfx950 mapping:
 //  * one workgroup of two wavefronts per kept row and level: each wavefront
@@ -26,9 +27,7 @@
 //    redundant readers never see a half-written block and the assembled
 //    blocks of eliminated rows stay untouched;
 //  * the last levels (few rows) run in one workgroup with barriers between
-//    levels, together with the top and their back-substitution;
-//  * the right-hand side can ride along with the factorisation (factor_solve),
-//    so a Newton step pays one launch per level plus one per back level.
+//    levels.
 // Blocks are m x m row-major with m <= 32; kernels work on MT = 16 or 32
 // (padding rows/columns get identity on B and zeros elsewhere).
 #include "gf_internal.h"
@@ -37,20 +36,11 @@
 
 namespace {
 
-typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 // 16x16x4 MFMA.  A(i, k) in lane i + 16 k, B(k, j) in lane j + 16 k; result item v
-// of lane l is row 4 v + l / 16 (f64) or 4 (l / 16) + v (f32), column l % 16.
+// of lane l is row 4 (l / 16) + v, column l % 16.
 template <typename T> struct mma;
-template <> struct mma<double> {
-    typedef v4d acc_t;
-    static __device__ __forceinline__ acc_t run(double a, double b, acc_t c)
-    {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int lane, int v) { return 4 * v + (lane >> 4); }
-};
 template <> struct mma<float> {
     typedef v4f acc_t;
     static __device__ __forceinline__ acc_t run(float a, float b, acc_t c)
@@ -60,12 +50,6 @@ template <> struct mma<float> {
     static __device__ __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }
 };
 
-__device__ __forceinline__ double rdl(double v, int l)
-{
-    int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
-}
 __device__ __forceinline__ float rdl(float v, int l)
 {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
@@ -86,11 +70,10 @@ template <int MT> struct cfg {
     static constexpr int PAIRS = MT == 16 ? 4 : 1;  // wave pairs of the tail workgroup
 };
 
-// Per wave pair LDS: eliminated neighbours [l, r] x [Binv, X, Y], kept row A_k, C_k, z_l, z_r.
+// Per wave pair LDS: eliminated neighbours [l, r] x [Binv, X, Y], kept row A_k, C_k.
 template <typename T, int MT> struct PairSmem {
     T e[2][3][cfg<MT>::BLK];
     T k[2][cfg<MT>::BLK];
-    T z[2][MT];
 };
 
 // Loads the augmented [B | I | A | C] of block row e into the wave's registers
@@ -180,7 +163,7 @@ template <typename T, int MT> __device__ void wave_gj(T (&col)[cfg<MT>::S][MT], 
 // and, when `to_global`, into Bi/X/Y of block row e.
 template <typename T, int MT>
 __device__ __forceinline__ void store_elim(const T (&col)[cfg<MT>::S][MT], T *sE, T *Bi, T *X, T *Y, int e, int m,
-                                           bool to_global, bool keep_bi)
+                                           bool to_global)
 {
     const int lane = threadIdx.x & 63;
     const size_t bs = (size_t)m * m, o = (size_t)e * bs;
@@ -193,7 +176,7 @@ __device__ __forceinline__ void store_elim(const T (&col)[cfg<MT>::S][MT], T *sE
 #pragma unroll
         for (int i = 0; i < MT; i++) {
             dst[i * cfg<MT>::LD + cc] = col[s][i];
-            if (to_global && (part != 1 || keep_bi) && i < m && cc < m) g[o + (size_t)i * m + cc] = col[s][i];
+            if (to_global && i < m && cc < m) g[o + (size_t)i * m + cc] = col[s][i];
         }
     }
 }
@@ -261,14 +244,10 @@ struct Fac {
 // (threads 128 wp .. 128 wp + 127 of the workgroup).  Every thread of the
 // workgroup must call it the same number of times (it holds barriers); pairs
 // with nothing to do pass active = false.
-// f: the right-hand side being reduced (null: factor only); zout: z of the
-// eliminated rows.
 // Every global read of the step (the eliminated neighbour's augmented row, the
-// kept row's couplings and diagonal block, both right-hand-side pieces) is
-// issued before the Gauss-Jordan sweep, so a step pays one memory round trip.
+// kept row's couplings and diagonal block) is issued before the Gauss-Jordan sweep, so a step pays one memory round trip.
 template <typename T, int MT>
-__device__ void fac_step(const Fac &F, PairSmem<T, MT> &sm, bool active, int L, int nL, int q, T *Lsv, T *Rsv,
-                         double *f, double *zout)
+__device__ void fac_step(const Fac &F, PairSmem<T, MT> &sm, bool active, int L, int nL, int q, T *Lsv, T *Rsv)
 {
     typedef typename mma<T>::acc_t acc_t;
     constexpr int NT = MT / 16, KV = MT * MT / 64;
@@ -282,9 +261,6 @@ __device__ void fac_step(const Fac &F, PairSmem<T, MT> &sm, bool active, int L, 
     const bool doE = active && (wv == 0 || hasR);
     const int e = wv == 0 ? l : r, pe = wv == 0 ? p - 1 : p + 1;
     const bool own = wv == 0 || p + 2 == nL;  // the right neighbour is written here only if it is the last row
-    // B^-1 and the kept-row couplings are stored only for later solve-only sweeps;
-    // a factorisation that reduces its right-hand side (f) needs X and Y alone.
-    const bool keep = f == nullptr;
 
     // ---- reads
     // (unconditional loads from clamped in-block addresses, selected afterwards;
@@ -323,14 +299,6 @@ __device__ void fac_step(const Fac &F, PairSmem<T, MT> &sm, bool active, int L, 
                 const int i = 16 * ti + mma<T>::row(lane, v), jj = 16 * tj + (lane & 15);
                 bk[ti][tj][v] = active && wv == 0 && i < m && jj < m ? bk[ti][tj][v] : T(0);
             }
-    // right-hand side pieces: f_e (staged for z_e, read for j < m only) and f_k
-    // (used by wave 0's lanes < m); lanes >= m hold a duplicate entry
-    double fe = 0.0, fk = 0.0;
-    if (f) {
-        const int li = lane < m ? lane : m - 1;
-        fe = f[(size_t)e * m + li];
-        fk = f[(size_t)k * m + li];
-    }
     T col[cfg<MT>::S][MT];  // (loaded by every wave: e is a valid row also when it is not eliminated here)
     load_aug<T, MT>(col, A, B, C, e, m, pe >= 1, pe + 1 < nL);
 
@@ -342,29 +310,18 @@ __device__ void fac_step(const Fac &F, PairSmem<T, MT> &sm, bool active, int L, 
         for (int jv = 0; jv < KV; jv++) {
             const int t = lane + 64 * jv, i = t / MT, jj = t % MT;
             dst[i * cfg<MT>::LD + jj] = kv[jv];
-            if (keep && i < m && jj < m) sv[(size_t)i * m + jj] = kv[jv];
+            if (i < m && jj < m) sv[(size_t)i * m + jj] = kv[jv];
         }
-        if (f && lane < MT) sm.z[wv][lane] = T(fe);
     }
     // ---- eliminated neighbour
     if (doE) {
         wave_gj<T, MT>(col, F.flag, m);
-        store_elim<T, MT>(col, &sm.e[wv][0][0], (T *)F.Bi, (T *)F.X, (T *)F.Y, e, m, own, keep);
+        store_elim<T, MT>(col, &sm.e[wv][0][0], (T *)F.Bi, (T *)F.X, (T *)F.Y, e, m, own);
     } else if (active) {
         // no right neighbour: zero X_r, Y_r so the products below need no special case
         for (int t = lane; t < 3 * cfg<MT>::BLK; t += 64) (&sm.e[1][0][0])[t] = T(0);
     }
     __syncthreads();
-    T zl = T(0);
-    if (active && f && lane < MT) {
-        // z of the eliminated neighbour: Binv_e f_e (f_e staged in sm.z)
-        if (doE && lane < m) {
-            // (the padding entries of B^-1 and z are zero: all MT terms are exact)
-#pragma unroll
-            for (int j = 0; j < MT; j++) zl += sm.e[wv][0][lane * cfg<MT>::LD + j] * sm.z[wv][j];
-            if (own) zout[(size_t)e * m + lane] = (double)zl;
-        }
-    }
     if (active) {
         if (wv == 0) {
             acc_t acc[NT][NT];
@@ -397,38 +354,21 @@ __device__ void fac_step(const Fac &F, PairSmem<T, MT> &sm, bool active, int L, 
             store_neg<T, MT>(acc, C + (size_t)k * bs, m);
         }
     }
-    __syncthreads();  // sm.z is overwritten with z below (all readers of f_e are done)
-    if (active && f && lane < MT) sm.z[wv][lane] = zl;
-    __syncthreads();
-    if (active && f && wv == 0 && lane < m) {
-        T s = T(0);
-#pragma unroll
-        for (int j = 0; j < MT; j++)
-            s += sm.k[0][lane * cfg<MT>::LD + j] * sm.z[0][j] + sm.k[1][lane * cfg<MT>::LD + j] * sm.z[1][j];
-        f[(size_t)k * m + lane] = fk - (double)s;
-    }
     __syncthreads();
 }
 
-// Top row (the single active row after the last level): Binv_top, and
-// zout_top = Binv_top f_top when f is given.  One wavefront (wave 0 of pair 0).
+// Top row (the single active row after the last level): Binv_top.  One wavefront
+// (wave 0 of pair 0).
 template <typename T, int MT>
-__device__ void top_step(const Fac &F, PairSmem<T, MT> &sm, int levels, const double *f, double *zout)
+__device__ void top_step(const Fac &F, PairSmem<T, MT> &sm, int levels)
 {
-    const int m = F.m, lane = threadIdx.x & 63;
+    const int m = F.m;
     const int e = lvl_row(0, levels);
     if (threadIdx.x < 64) {
         T col[cfg<MT>::S][MT];
         load_aug<T, MT>(col, (const T *)F.A, (const T *)F.B, (const T *)F.C, e, m, false, false);
         wave_gj<T, MT>(col, F.flag, m);
-        store_elim<T, MT>(col, &sm.e[0][0][0], (T *)F.Bi, (T *)F.X, (T *)F.Y, e, m, true, f == nullptr);
-        if (f && lane < m) {
-            T s = T(0);
-#pragma unroll
-            for (int j = 0; j < MT; j++)
-                if (j < m) s += sm.e[0][0][lane * cfg<MT>::LD + j] * (T)f[(size_t)e * m + (j < m ? j : 0)];
-            zout[(size_t)e * m + lane] = (double)s;
-        }
+        store_elim<T, MT>(col, &sm.e[0][0][0], (T *)F.Bi, (T *)F.X, (T *)F.Y, e, m, true);
     }
     __syncthreads();
 }
@@ -475,22 +415,16 @@ __device__ __forceinline__ void back_rows(const T *X, const T *Y, int m, int L, 
 
 // ---- factor kernels -----------------------------------------------------------
 template <typename T, int MT>
-__global__ __launch_bounds__(128) void btd_level_kernel(Fac F, int L, int nL, T *Lsv, T *Rsv, double *f,
-                                                        double *zout)
+__global__ __launch_bounds__(128) void btd_level_kernel(Fac F, int L, int nL, T *Lsv, T *Rsv)
 {
     __shared__ PairSmem<T, MT> sm;
-    fac_step<T, MT>(F, sm, true, L, nL, blockIdx.x, Lsv, Rsv, f, zout);
+    fac_step<T, MT>(F, sm, true, L, nL, blockIdx.x, Lsv, Rsv);
 }
 
-// Levels L0 .. levels-1, the top and (with f) the back-substitution of levels
-// levels-1 .. Lb (Lb <= L0: the upper levels below the tail have so few
-// eliminated rows that their back-substitution costs less here than a launch),
-// in one workgroup of PAIRS wave pairs.  nblk: block rows of level 0 (level L
-// has nblk >> L active rows).
+// Levels L0 .. levels-1 and the top, in one workgroup of PAIRS wave pairs.
 template <typename T, int MT>
 __global__ __launch_bounds__(128 * cfg<MT>::PAIRS) void btd_tail_kernel(Fac F, int L0, int levels, int nL0,
-                                                                        T *Lsv, T *Rsv, const long long *save,
-                                                                        double *f, double *x, int Lb, int nblk)
+                                                                        T *Lsv, T *Rsv, const long long *save)
 {
     constexpr int PAIRS = cfg<MT>::PAIRS;
     __shared__ PairSmem<T, MT> sm[PAIRS];
@@ -501,17 +435,11 @@ __global__ __launch_bounds__(128 * cfg<MT>::PAIRS) void btd_tail_kernel(Fac F, i
         for (int base = 0; base < nk; base += PAIRS) {
             const int q = base + wp;
             fac_step<T, MT>(F, sm[wp], q < nk, L, nL, q < nk ? q : 0, Lsv + save[L] * (size_t)F.m * F.m,
-                            Rsv + save[L] * (size_t)F.m * F.m, f, x);
+                            Rsv + save[L] * (size_t)F.m * F.m);
         }
         nL /= 2;
     }
-    top_step<T, MT>(F, sm[0], levels, f, x);
-    if (!f) return;
-    // back-substitution of levels levels-1 .. Lb
-    for (int L = levels - 1; L >= Lb; L--) {
-        back_rows<T, MT>((const T *)F.X, (const T *)F.Y, F.m, L, nblk >> L, x, threadIdx.x, blockDim.x);
-        __syncthreads();
-    }
+    top_step<T, MT>(F, sm[0], levels);
 }
 
 // ---- solve-only kernels (factors already in place) ------------------------------
@@ -595,19 +523,10 @@ __global__ __launch_bounds__(256) void btd_back_kernel(const T *X, const T *Y, i
 
 }  // namespace
 
-// Level structure of the cyclic reduction (no device call).  Returns the number
-// of saved coupling blocks (the Lsv / Rsv extent).
-int gf_btd_plan(gf_btd &b, int m, int nblk, int elem_size)
+// Level structure of the kept factors.
+static void btd_plan(gf_btd &b, int m, int nblk)
 {
-    if (m < 1 || m > 32) {
-        gf_set_error("block-tridiagonal solver: block size out of range");
-        return GF_E_UNSUPPORTED;
-    }
-    b.m = m;
     b.mt = m <= 16 ? 16 : 32;
-    b.nblk = nblk;
-    b.bsz = (size_t)m * m;
-    b.elem_size = elem_size;
     b.lvl_n.clear();
     b.lvl_save.clear();
     const int tail_rows = b.mt == 16 ? 16 : 4;  // 4 x the tail workgroup's wave pairs
@@ -624,23 +543,28 @@ int gf_btd_plan(gf_btd &b, int m, int nblk, int elem_size)
     }
     b.levels = L;
     if (b.tail_level < 0) b.tail_level = L;
-    // the back-substitution of the levels above the tail runs as one wide launch
-    // per level: inside the single tail workgroup it took longer than the launches
-    b.back_level = b.tail_level;
     b.n_save = (long long)save;
-    return GF_OK;
 }
 
 int gf_btd_alloc(gf_btd &b, int m, int nblk, int elem_size)
 {
-    GF_TRY(gf_btd_plan(b, m, nblk, elem_size));
-    const size_t save = (size_t)b.n_save;
+    if (m < 1 || m > 32) {
+        gf_set_error("block-tridiagonal solver: block size out of range");
+        return GF_E_UNSUPPORTED;
+    }
+    b.m = m;
+    b.nblk = nblk;
+    b.bsz = (size_t)m * m;
+    b.elem_size = elem_size;
     size_t blocks = (size_t)nblk * b.bsz * elem_size;
-    size_t sv = (save ? save : 1) * b.bsz * elem_size;
     // A, B, C contiguous: the assembly clears them with one fill
     GF_TRY(gf_pool_alloc(&b.A, 3 * blocks));
     b.B = (char *)b.A + blocks;
     b.C = (char *)b.A + 2 * blocks;
+    if (elem_size == 8) return gf_pool_alloc((void **)&b.cr_work, gf_cr_plan(b, m, nblk) * 8);
+    btd_plan(b, m, nblk);
+    const size_t save = (size_t)b.n_save;
+    size_t sv = (save ? save : 1) * b.bsz * elem_size;
     void **arrs[] = {&b.Bi, &b.X, &b.Y};
     for (void **a : arrs) GF_TRY(gf_pool_alloc(a, blocks));
     GF_TRY(gf_pool_alloc(&b.Lsv, sv));
@@ -657,14 +581,15 @@ int gf_btd_alloc(gf_btd &b, int m, int nblk, int elem_size)
 
 void gf_btd_free(gf_btd &b)
 {
-    void *arrs[] = {b.A, b.Bi, b.X, b.Y, b.Lsv, b.Rsv, b.d_save};  // B and C live inside A's allocation
+    void *arrs[] = {b.A, b.Bi, b.X, b.Y, b.Lsv, b.Rsv, b.d_save, b.cr_work};  // B and C live inside A's allocation
     for (void *a : arrs) gf_pool_free(a);
     b.A = b.B = b.C = b.Bi = b.X = b.Y = b.Lsv = b.Rsv = nullptr;
     b.d_save = nullptr;
+    b.cr_work = nullptr;
 }
 
 template <typename T, int MT>
-static int btd_factor_t(gf_btd &b, hipStream_t s, int *d_flag, double *f, double *x)
+static int btd_factor_t(gf_btd &b, hipStream_t s, int *d_flag)
 {
     Fac F{b.A, b.B, b.C, b.Bi, b.X, b.Y, b.m, d_flag};
     T *Lsv = (T *)b.Lsv, *Rsv = (T *)b.Rsv;
@@ -672,51 +597,20 @@ static int btd_factor_t(gf_btd &b, hipStream_t s, int *d_flag, double *f, double
     int launches = 0;
     for (int L = 0; L < b.tail_level; L++) {
         const int nL = b.lvl_n[L];
-        const int pr = gf_probe_begin(s, GF_KC_BTD_LEVEL);
         hipLaunchKernelGGL((btd_level_kernel<T, MT>), dim3(nL / 2), dim3(128), 0, s, F, L, nL, Lsv + b.lvl_save[L] * bs,
-                           Rsv + b.lvl_save[L] * bs, f, x);
-        gf_probe_end(s, pr, nL / 2);
+                           Rsv + b.lvl_save[L] * bs);
         launches++;
     }
     const int nL0 = b.tail_level < b.levels ? b.lvl_n[b.tail_level] : 1;
-    const int pr = gf_probe_begin(s, GF_KC_BTD_TAIL);
     hipLaunchKernelGGL((btd_tail_kernel<T, MT>), dim3(1), dim3(128 * cfg<MT>::PAIRS), 0, s, F, b.tail_level, b.levels,
-                       nL0, Lsv, Rsv, (const long long *)b.d_save, f, x, b.back_level, b.nblk);
-    gf_probe_end(s, pr, nL0);
-    launches++;
-    if (f) {
-        for (int L = b.back_level - 1; L >= 0; L--) {
-            const int nL = b.lvl_n[L];
-            const int work = (nL + 1) / 2 * b.m;
-            hipLaunchKernelGGL((btd_back_kernel<T, MT>), dim3((work + 255) / 256), dim3(256), 0, s, (const T *)b.X,
-                               (const T *)b.Y, b.m, L, nL, x);
-            launches++;
-        }
-    }
+                       nL0, Lsv, Rsv, (const long long *)b.d_save);
     GF_HIP(hipGetLastError());
-    return launches;
-}
-
-template <typename T> static int btd_factor_dispatch(gf_btd &b, hipStream_t s, int *d_flag, double *f, double *x)
-{
-    return b.mt == 16 ? btd_factor_t<T, 16>(b, s, d_flag, f, x) : btd_factor_t<T, 32>(b, s, d_flag, f, x);
+    return launches + 1;
 }
 
 int gf_btd_factor(gf_btd &b, hipStream_t s, int *d_flag)
 {
-    if (b.elem_size == 8) return btd_factor_dispatch<double>(b, s, d_flag, nullptr, nullptr);
-    return btd_factor_dispatch<float>(b, s, d_flag, nullptr, nullptr);
-}
-
-int gf_btd_factor_solve(gf_btd &b, hipStream_t s, int *d_flag, const double *rhs, double *x, int n, double *work)
-{
-    if (rhs == x || work == x) {
-        gf_set_error("block-tridiagonal factor_solve: x must differ from rhs and work");
-        return GF_E_ARG;
-    }
-    if (rhs != work) GF_HIP(hipMemcpyAsync(work, rhs, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice, s));
-    if (b.elem_size == 8) return btd_factor_dispatch<double>(b, s, d_flag, work, x);
-    return btd_factor_dispatch<float>(b, s, d_flag, work, x);
+    return b.mt == 16 ? btd_factor_t<float, 16>(b, s, d_flag) : btd_factor_t<float, 32>(b, s, d_flag);
 }
 
 template <typename T, int MT> static int btd_solve_t(gf_btd &b, hipStream_t s, double *f, double *x)
@@ -754,7 +648,5 @@ int gf_btd_solve(gf_btd &b, hipStream_t s, const double *rhs, double *x, int n, 
         return GF_E_ARG;
     }
     if (rhs != work) GF_HIP(hipMemcpyAsync(work, rhs, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice, s));
-    if (b.elem_size == 8)
-        return b.mt == 16 ? btd_solve_t<double, 16>(b, s, work, x) : btd_solve_t<double, 32>(b, s, work, x);
     return b.mt == 16 ? btd_solve_t<float, 16>(b, s, work, x) : btd_solve_t<float, 32>(b, s, work, x);
 }

@@ -255,21 +255,28 @@ enum { SG_PER_GP = 21, SG_COUNT = 63 };  // per gp: Q_i 9, kr1 3, kr2 3, zx1 3, 
 // Nodal loads grouped by node (one device thread per loaded node).
 enum { NL_KIND = 0, NL_CS = 1, NL_MULT = 10, NL_TAB0 = 16, NL_TABN = 17, NL_REC = 18 };
 
-// Block-tridiagonal factor workspace (cyclic reduction), precision T.
+// Block-tridiagonal systems (cyclic reduction).  FP64 (elem_size 8): factored
+// and solved in one pass over chunks of block rows (gf_cr.hip), which leaves A, B
+// and C as they are.  FP32 (elem_size 4): factors kept for the refinement's
+// sweeps, one launch per level (gf_btd.hip).
 struct gf_btd {
-    int m = 0, mt = 16, nblk = 0, levels = 0, tail_level = 0;
-    int back_level = 0;             // lowest level whose back-substitution the tail kernel does
+    int m = 0, nblk = 0;
     size_t bsz = 0;                 // m*m
-    void *A = nullptr, *B = nullptr, *C = nullptr;     // [nblk][m][m] assembled blocks (kept rows reduced in place)
+    int elem_size = 8;
+    void *A = nullptr, *B = nullptr, *C = nullptr;     // [nblk][m][m] blocks (FP32: kept rows reduced in place)
+    // FP64
+    std::vector<int> cr_n, cr_R;    // block rows and rows of a chunk at each level
+    double *cr_work = nullptr;      // gf_cr_plan doubles
+    // FP32
+    int mt = 16, levels = 0, tail_level = 0;
     void *Bi = nullptr, *X = nullptr, *Y = nullptr;    // eliminated rows: B^-1, B^-1 A, B^-1 C
     void *Lsv = nullptr, *Rsv = nullptr;               // pre-update A_k, C_k per (level, kept row)
     long long *d_save = nullptr;    // lvl_save on the device
     std::vector<int> lvl_n;         // rows active at each level
     std::vector<long long> lvl_save; // offsets (in blocks) into Lsv/Rsv per level
     long long n_save = 0;           // saved coupling blocks over all levels
-    int elem_size = 8;
 };
-int gf_btd_plan(gf_btd &b, int m, int nblk, int elem_size);  // level structure only, no device call
+size_t gf_cr_plan(gf_btd &b, int m, int nblk);
 
 // Nested-dissection multifrontal factorisation (gf_nd.cpp plans it on the host,
 // gf_front.hip runs it).  Supernodes are the parts and separators of a recursive
@@ -356,7 +363,7 @@ int gf_front_solve(const gf_fronts &fp, int elem_size, const void *F, const void
 struct gf_kprobe {
     unsigned mask = 0;
     std::vector<hipEvent_t> ev;    // 2 per slot
-    std::vector<int> cls;
+    std::vector<int> cls, count;
     std::vector<double> units;
     int used = 0;
     double ms[GF_NKC] = {}, units_done[GF_NKC] = {};
@@ -365,7 +372,7 @@ struct gf_kprobe {
 
     bool wants(int c) const { return (mask >> c) & 1u; }
     int begin(hipStream_t s, int c);           // before the launch; -1 when not probed
-    void end(hipStream_t s, int slot, double units);
+    void end(hipStream_t s, int slot, double units, int count);
     int flush();                               // waits for the recorded pairs, accumulates
     ~gf_kprobe();
 };
@@ -377,9 +384,10 @@ struct gf_probe_scope {
     ~gf_probe_scope() { gf_probe = prev; }
 };
 inline int gf_probe_begin(hipStream_t s, int c) { return gf_probe && gf_probe->wants(c) ? gf_probe->begin(s, c) : -1; }
-inline void gf_probe_end(hipStream_t s, int slot, double units)
+// count: launches the bracket stands for in the class's tally
+inline void gf_probe_end(hipStream_t s, int slot, double units, int count = 1)
 {
-    if (slot >= 0) gf_probe->end(s, slot, units);
+    if (slot >= 0) gf_probe->end(s, slot, units, count);
 }
 
 // scalar block of a model (doubles): increment norms, failure flag, residual
@@ -559,12 +567,13 @@ int gf_node_commit(gf_model *m);
 
 int gf_btd_alloc(gf_btd &b, int m, int nblk, int elem_size);
 void gf_btd_free(gf_btd &b);
-// Both return the number of kernel launches issued (>= 0) or a negative status.
+// All return the number of kernel launches issued (>= 0) or a negative status.
+// FP32: factorisation, then x = K^-1 rhs with the factors in place (work: n
+// entries, may alias rhs, not x).
 int gf_btd_factor(gf_btd &b, hipStream_t s, int *d_flag);
-// x = K^-1 rhs (factors in place); work: n entries, may alias rhs, not x
 int gf_btd_solve(gf_btd &b, hipStream_t s, const double *rhs, double *x, int n, double *work);
-// factorisation with the right-hand side reduced alongside: x = K^-1 rhs
-int gf_btd_factor_solve(gf_btd &b, hipStream_t s, int *d_flag, const double *rhs, double *x, int n, double *work);
+// FP64: factorisation and x = K^-1 rhs in one pass.
+int gf_btd_factor_solve(const gf_btd &b, hipStream_t s, int *d_flag, const double *rhs, double *x);
 
 // Asynchronous halves of gf_assemble and gf_solve + gf_update: *_enqueue puts the
 // work on the model's stream, *_result reads the norms once the stream passed it.

@@ -261,7 +261,7 @@ int gf_mixed_fallback(gf_model *m)
 {
     const int npad = m->npad;
     GF_TRY(gf_launch_fill_bytes(m->stream, m->d_flag, 4));
-    if (m->layout == GM_BTD) return gf_btd_factor_solve(m->btd, m->stream, m->d_flag, m->d_r, m->d_x, npad, m->d_res);
+    if (m->layout == GM_BTD) return gf_btd_factor_solve(m->btd, m->stream, m->d_flag, m->d_r, m->d_x);
     if (m->fronts_on) {
         const int l = gf_front_factor(m->fronts, 8, m->d_band, m->band_ld, m->half_band, nullptr, m->d_front,
                                       m->d_front_e, m->stream, m->d_flag, m->d_r, m->d_front_v);

@@ -98,6 +98,7 @@ int gf_kprobe::begin(hipStream_t s, int c)
         ev.push_back(a);
         ev.push_back(b);
         cls.push_back(0);
+        count.push_back(0);
         units.push_back(0.0);
     }
     const int slot = used++;
@@ -106,9 +107,10 @@ int gf_kprobe::begin(hipStream_t s, int c)
     return slot;
 }
 
-void gf_kprobe::end(hipStream_t s, int slot, double u)
+void gf_kprobe::end(hipStream_t s, int slot, double u, int n)
 {
     units[slot] = u;
+    count[slot] = n;
     (void)hipEventRecord(ev[2 * slot + 1], s);
 }
 
@@ -121,7 +123,7 @@ int gf_kprobe::flush()
         GF_HIP(hipEventElapsedTime(&t, ev[2 * i], ev[2 * i + 1]));
         ms[cls[i]] += t;
         units_done[cls[i]] += units[i];
-        launches[cls[i]]++;
+        launches[cls[i]] += count[i];
     }
     used = 0;
     return GF_OK;
@@ -500,8 +502,11 @@ static size_t footprint(const gf_model_desc *d, const gf_model *m, int precision
     b += 3 * npad * 8 + 256;                                                   // r, x, work, scalars
     size_t tangent;
     if (m->layout == GM_BTD) {
-        size_t blocks = 6 * (size_t)nblk + 2 * (size_t)nblk;                  // A B C Bi X Y + saved couplings
-        tangent = blocks * (size_t)bm * bm;
+        gf_btd t;
+        const size_t bs = (size_t)bm * bm;
+        b += (3 * (size_t)nblk * bs + gf_cr_plan(t, bm, nblk)) * 8;           // A B C, eliminated and reduced rows
+        if (precision == GF_PREC_MIXED) b += 8 * (size_t)nblk * bs * 4 + 3 * npad * 8;  // and Bi X Y, saved couplings
+        return b;
     } else if (m->fronts_on) {
         const gf_fronts &fp = m->fronts;
         const size_t factor = (size_t)(fp.f_elems + fp.e_elems);
@@ -1388,7 +1393,7 @@ static int solve_fp64_launches(gf_model *m, int &nl_fac, int &nl_sol)
         return nl_sol < 0 ? nl_sol : GF_OK;
     }
     if (m->layout == GM_BTD)
-        nl_fac = gf_btd_factor_solve(m->btd, m->stream, m->d_flag, m->d_r, m->d_x, (int)npad, m->d_swork);
+        nl_fac = gf_btd_factor_solve(m->btd, m->stream, m->d_flag, m->d_r, m->d_x);
     else nl_fac = gf_band_factor(m->d_band, 8, m->npad, m->half_band, m->stream, m->d_flag, m->d_band_inv);
     if (nl_fac < 0) return nl_fac;
     if (m->layout != GM_BTD) {
@@ -1727,7 +1732,7 @@ extern "C" int gf_btdsystem(int m, int nblk, const double *A, const double *B, c
     *info_fail = 0;
     const size_t bs = (size_t)m * m, blocks = (size_t)nblk * bs, n = (size_t)nblk * m;
     gf_btd t;
-    double *d_r = nullptr, *d_x = nullptr, *d_w = nullptr;
+    double *d_r = nullptr, *d_x = nullptr;
     int *d_flag = nullptr;
     hipStream_t s = nullptr;
     int flag = 0;
@@ -1736,17 +1741,13 @@ extern "C" int gf_btdsystem(int m, int nblk, const double *A, const double *B, c
         GF_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
         GF_HIP(hipMalloc(&d_r, n * 8));
         GF_HIP(hipMalloc(&d_x, n * 8));
-        GF_HIP(hipMalloc(&d_w, n * 8));
         GF_HIP(hipMalloc(&d_flag, 4));
         GF_TRY(gf_launch_fill_bytes(s, d_flag, 4));
         GF_HIP(hipMemcpyAsync(t.A, A, blocks * 8, hipMemcpyHostToDevice, s));
         GF_HIP(hipMemcpyAsync(t.B, B, blocks * 8, hipMemcpyHostToDevice, s));
         GF_HIP(hipMemcpyAsync(t.C, C, blocks * 8, hipMemcpyHostToDevice, s));
-        // the couplings past either end do not exist
-        GF_HIP(hipMemsetAsync(t.A, 0, bs * 8, s));
-        GF_HIP(hipMemsetAsync((double *)t.C + (blocks - bs), 0, bs * 8, s));
         GF_HIP(hipMemcpyAsync(d_r, b, n * 8, hipMemcpyHostToDevice, s));
-        int l = gf_btd_factor_solve(t, s, d_flag, d_r, d_x, (int)n, d_w);
+        int l = gf_btd_factor_solve(t, s, d_flag, d_r, d_x);
         if (l < 0) return l;
         GF_HIP(hipMemcpyAsync(x, d_x, n * 8, hipMemcpyDeviceToHost, s));
         GF_HIP(hipMemcpyAsync(&flag, d_flag, 4, hipMemcpyDeviceToHost, s));
@@ -1755,7 +1756,7 @@ extern "C" int gf_btdsystem(int m, int nblk, const double *A, const double *B, c
     };
     const int st = run();
     if (s) (void)hipStreamSynchronize(s);
-    void *bufs[] = {d_r, d_x, d_w, d_flag};
+    void *bufs[] = {d_r, d_x, d_flag};
     for (void *p : bufs)
         if (p) (void)hipFree(p);
     gf_btd_free(t);

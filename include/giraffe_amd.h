@@ -269,8 +269,10 @@ int gf_timing_read(gf_model *m, double *ms_out, long long *launches_out, int res
  * timing is enabled, every launch of a kernel class whose bit is set in `mask`
  * is bracketed by HIP events on the model's stream.  Read per class:
  * accumulated milliseconds, launches, and work units (GF_KC_* comments). */
-#define GF_KC_BTD_LEVEL      0  /* btd_level_kernel; unit: block row eliminated     */
-#define GF_KC_BTD_TAIL       1  /* btd_tail_kernel; unit: block row eliminated      */
+#define GF_KC_BTD_LEVEL      0  /* cr_reduce_kernel<, , false>; unit: block row eliminated,
+                                   counted in halvings of the rows down to 16 (a launch
+                                   runs three to five)                              */
+#define GF_KC_BTD_TAIL       1  /* cr_reduce_kernel<, , true>; unit: block row eliminated */
 #define GF_KC_BAND_PANEL     2  /* band_batch_inv_kernel; unit: flop of the batch inverses */
 #define GF_KC_BAND_UPDATE    3  /* band_step_kernel; unit: band column eliminated   */
 #define GF_KC_BAND_SWEEP     4  /* band_batch_apply_kernel, band_couple_kernel; unit: row
@@ -353,7 +355,7 @@ int gf_btdsystem(int m, int nblk, const double *A, const double *B, const double
  * and info_fail are device pointers (info_fail: one int, written 0 or 1); the
  * work is enqueued on `stream` (a hipStream_t, NULL for the null stream) and
  * the call returns without waiting.  The factor workspace lives in a fixed
- * device array of the library (9.4 MB on each GPU it runs on, held until the
+ * device array of the library (4.2 MB on each GPU it runs on, held until the
  * process ends): nblk * m * m <= 131072, else GF_E_CAPACITY before any device
  * work.  Calls that overlap on one GPU share that array and race. */
 int gf_btdsystem_noalloc(int m, int nblk, const double *A, const double *B, const double *C, const double *b,
