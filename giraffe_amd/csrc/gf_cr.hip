@@ -61,16 +61,6 @@ template <int H, int R> struct CrSmem {
     double x[R + 1][MT];
 };
 
-// Lanes i == K of every DPP row, as a wavefront mask.  Formed in place by one
-// scalar instruction: as a compare or a constant the compiler keeps all sixteen,
-// which the scalar registers do not hold.
-template <int K> __device__ __forceinline__ unsigned long long lanes_at()
-{
-    unsigned long long v;
-    asm volatile("s_lshl_b64 %0, %1, %2" : "=s"(v) : "s"(0x0001000100010001ull), "n"(K) : "scc");
-    return v;
-}
-
 // Interchange of row K with the largest row of column K (rows >= K), when the
 // pivot is less than half of it.  Rare and wave-uniform.
 template <int H, int NC, int K>

@@ -266,6 +266,15 @@ __device__ __forceinline__ void nb_pivot(double *r, double h, double &p, double 
               GF_R(10), GF_R(11), GF_R(12), GF_R(13), GF_R(14), GF_R(15), GF_R(16), GF_R(17), GF_R(18),
               GF_R(19), GF_R(20), GF_R(21), GF_R(22), GF_R(23), GF_POUT GF_PIN);
 }
+// The same for 15 columns without the compare.
+template <int K> __device__ __forceinline__ void nb_pivot15(double *r, double h, double &ip, double &g)
+{
+    double p, t;
+    asm("s_nop 1\n\t" GF_F(0) GF_F(1) GF_F(2) GF_PMOV GF_F(3) GF_F(4) "v_rcp_f64 %[ip], %[p]\n\t" GF_F(5) GF_F(6)
+            GF_F(7) GF_PE1 GF_F(8) GF_PE2 GF_F(9) GF_F(10) GF_PE3 GF_F(11) GF_F(12) GF_PG_NL GF_F(13) GF_F(14)
+        : GF_R(0), GF_R(1), GF_R(2), GF_R(3), GF_R(4), GF_R(5), GF_R(6), GF_R(7), GF_R(8), GF_R(9), GF_R(10),
+          GF_R(11), GF_R(12), GF_R(13), GF_R(14), [p] "=&v"(p), [ip] "=&v"(ip), [t] "=&v"(t), [g] "=&v"(g) GF_PIN);
+}
 #undef GF_F
 #undef GF_R
 #undef GF_PMOV
@@ -280,5 +289,15 @@ __device__ __forceinline__ void nb_pivot(double *r, double h, double &p, double 
 #undef GF_PIN
 
 #undef GF_NB
+
+// Lanes i == K of every DPP row, as a wavefront mask.  Formed in place by one
+// scalar instruction: as a compare or a constant the compiler keeps all sixteen,
+// which the scalar registers do not hold.
+template <int K> __device__ __forceinline__ unsigned long long lanes_at()
+{
+    unsigned long long v;
+    asm volatile("s_lshl_b64 %0, %1, %2" : "=s"(v) : "s"(0x0001000100010001ull), "n"(K) : "scc");
+    return v;
+}
 
 }  // namespace

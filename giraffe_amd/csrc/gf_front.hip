@@ -75,7 +75,7 @@ template <typename T> struct AsmSmem {
 constexpr int ASM_T = 512, ASM_R = NB * NB / ASM_T;
 
 template <typename T>
-__global__ __launch_bounds__(ASM_T) void front_assemble_kernel(FrontTab t, int first, const double *ab, int ld, int hb,
+__global__ __launch_bounds__(ASM_T, 6) void front_assemble_kernel(FrontTab t, int first, const double *ab, int ld, int hb,
                                                                const double *D, T *Fb, T *Eb, int *flag,
                                                                const double *rhs, double *Vb)
 {

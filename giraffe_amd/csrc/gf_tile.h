@@ -4,7 +4,7 @@
 // 64 x 64 block inverse with pivot perturbation, row-major tile transfers.
 // Device code only; every definition has internal linkage.
 #pragma once
-#include "gf_internal.h"
+#include "gf_dpp.h"
 
 namespace {
 
@@ -218,13 +218,65 @@ __device__ __forceinline__ void inv16_pivot(T (&a)[4], T &sc, int i, int q, cons
     if constexpr (K + 1 < 16) inv16_pivot<T, K + 1>(a, sc, i, q, ieps, huge, bad, pert);
 }
 
+// FP64: the same inverse with every lane holding the whole of its row (the four
+// DPP rows hold copies), so that a row's multiplier is its own lane's and the
+// pivot row comes inside the multiply-add: about 27 instructions a pivot against
+// 70, with the next pivot's reciprocal formed among them.  Pivots are taken as
+// they are; sc (their reciprocals, row by row) tells at the end whether one was
+// below its threshold or not finite.
+template <int K>
+__device__ __forceinline__ void inv16_row_pivot(double (&a)[16], double &sc, double ip, double g)
+{
+    const bool isk = __builtin_amdgcn_inverse_ballot_w64(lanes_at<K>());
+    const double h = isk ? 0.0 : g;
+    sc = isk ? ip : sc;
+    a[K] = __hiloint2double(isk ? 0x3ff00000 : __double2hiint(h), __double2loint(h));  // row K: 1, else -a(i, K) / p
+    double t[15];
+#pragma unroll
+    for (int j = 0; j < 15; j++) t[j] = a[(K + 1 + j) & 15];
+    if constexpr (K + 1 < 16) nb_pivot15<K>(t, h, ip, g);
+    else nb_self<K, 15>(t, h);
+#pragma unroll
+    for (int j = 0; j < 15; j++) a[(K + 1 + j) & 15] = t[j];
+    if constexpr (K + 1 < 16) inv16_row_pivot<K + 1>(a, sc, ip, g);
+}
+__device__ __forceinline__ bool inv16_rows(double *b, const double *ieps, double huge)
+{
+    const int lane = threadIdx.x & 63, i = lane & 15;
+    double a[16], sc = 1.0;
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) {
+        const double2 w = *reinterpret_cast<const double2 *>(b + i * LDT + e);
+        a[e] = w.x;
+        a[e + 1] = w.y;
+    }
+    const double ie = ieps[i], p0 = nb_get<0>(a[0]), ip0 = pivot_rcp(p0);
+    inv16_row_pivot<0>(a, sc, ip0, -(a[0] * ip0));
+    // |p| >= eps and |p| < huge for every pivot p = 1 / sc
+    const double as = fabs(sc);
+    if (__any(!(as <= ie && as * huge > 1.0))) return false;
+    if (lane < 16) {
+#pragma unroll
+        for (int e = 0; e < 16; e += 2) {
+            double2 w;
+            w.x = sc * a[e];
+            w.y = sc * a[e + 1];
+            *reinterpret_cast<double2 *>(b + i * LDT + e) = w;
+        }
+    }
+    return true;
+}
+__device__ __forceinline__ bool inv16_rows(float *, const float *, float) { return false; }
+
 // One wavefront: in-place Gauss-Jordan inverse (no interchanges) of the 16 x 16
 // block at b (stride LDT); the 16 pivots run in registers with DPP and
 // permlane moves, no barrier and no LDS access on the pivot chain.  ieps: the
-// reciprocals of the sixteen pivot thresholds (LDS).
+// reciprocals of the sixteen pivot thresholds (LDS).  FP64 blocks come here only
+// where inv16_rows met a pivot that has to be replaced.
 template <typename T>
 __device__ __forceinline__ void inv16(T *b, const T *ieps, T huge, bool &bad, bool &pert)
 {
+    if (__builtin_expect(inv16_rows(b, ieps, huge), 1)) return;
     const int lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
     T a[4], sc = T(1);
 #pragma unroll
@@ -246,17 +298,28 @@ __device__ __forceinline__ typename mfma<T>::acc_t mm16(const T *P, int lp, cons
     return acc;
 }
 
-// Scratch of inverse64: two sets of three saved 16 x 16 column blocks.
-constexpr int INV_TMP = 2 * 3 * 16 * TMP_LD;
+// Scratch of inverse64: two sets of three saved 16 x 16 column blocks, and one
+// more block.
+constexpr int INV_TMP = (2 * 3 + 1) * 16 * TMP_LD;
+
+// LDS writes of a wavefront before its own later reads.
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 // In-place inverse of the 64 x 64 matrix M ([64][LDT]) by 256 threads: block
 // Gauss-Jordan over 16 x 16 blocks.  Step kb, with the pivot block P already
-// inverted in place and the column blocks C_i = M(i, kb) (i != kb) saved: waves
-// 0-2 form the row blocks R_j = P^-1 M(kb, j); then the four waves update
-// M(i, j) -= C_i R_j and set M(i, kb) = -C_i P^-1 (MFMA 16x16x4).  The next
-// pivot block is updated first, by wave 0, which then inverts it (inv16) while
-// waves 1-3 finish the step's other blocks and save the next step's column
-// blocks: two barriers per step.  No interchanges: a pivot smaller than 1e-13
+// inverted in place and the column blocks C_i = M(i, kb) (i != kb) saved: row
+// blocks R_j = P^-1 M(kb, j), M(i, j) -= C_i R_j, M(i, kb) = -C_i P^-1 (MFMA
+// 16x16x4).  The chain is the next pivot block: wave 0 forms its R itself,
+// updates that block and inverts it (inv16) while waves 1-3 each take a column
+// (its R, then its blocks; wave 3 the rest of the next pivot's column, which it
+// saves for the next step, and the pivot column), so no wave needs another's
+// result within a step: one barrier per step.  M(kb, kb + 1) itself keeps its
+// old value (the next step overwrites it from the saved blocks).  No
+// interchanges: a pivot smaller than 1e-13
 // (FP32: 1e-6) of its row's original diagonal entry (of the block's largest
 // entry where that is zero) -- a threshold that does not depend on how rows and
 // columns are scaled -- is replaced by that size with its sign (bit 2 of
@@ -293,64 +356,78 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
             const T dk = ie[lane];
             ie[lane] = rcp_of<T>(pg.rel * (dk > T(0) ? dk : mx));
         }
+        wave_lds_fence();
         inv16<T>(M + 16 * kb * LDT + 16 * kb, ie, pg.huge, bad, pert);
     };
     constexpr int CS = 16 * TMP_LD, CB = 3 * CS;  // one saved block, one set
+    auto block = [&](int i, int j) { return M + 16 * i * LDT + 16 * j; };
+    auto put = [&](T *dst, int ld, const typename mfma<T>::acc_t &v) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) dst[mfma<T>::row(lane, e) * ld + (lane & 15)] = v[e];
+    };
+    // M(i, j) -= C R (saved copy to sv when given)
+    auto update = [&](int i, int j, const T *Ci, const T *R, int ldr, T *sv) {
+        T *Mij = block(i, j);
+        const typename mfma<T>::acc_t acc = mm16<T>(Ci, TMP_LD, R, ldr);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int r = mfma<T>::row(lane, e), c = lane & 15;
+            const T x = Mij[r * LDT + c] - acc[e];
+            Mij[r * LDT + c] = x;
+            if (sv) sv[r * TMP_LD + c] = x;
+        }
+    };
     // step 0's pivot block and column blocks
     if (wave == 0) {
         pivot_block(0);
     } else if (act) {
-        const T *src = M + 16 * wave * LDT;
+        const T *src = block(wave, 0);
         for (int t = lane; t < 256; t += 64) tmp[(wave - 1) * CS + (t >> 4) * TMP_LD + (t & 15)] = src[(t >> 4) * LDT + (t & 15)];
     }
     __syncthreads();
+#pragma unroll 1
     for (int kb = 0; kb < 4; kb++) {
-        const T *cur = tmp + (kb & 1) * CB;
+        const T *cur = tmp + (kb & 1) * CB, *P = block(kb, kb);
         T *nxt = tmp + ((kb + 1) & 1) * CB;
-        T *P = M + 16 * kb * LDT + 16 * kb;
-        if (wave < 3) {
-            T *R = M + 16 * kb * LDT + 16 * (wave < kb ? wave : wave + 1);
-            const typename mfma<T>::acc_t acc = mm16<T>(P, LDT, R, LDT);
-#pragma unroll
-            for (int v = 0; v < 4; v++) R[mfma<T>::row(lane, v) * LDT + (lane & 15)] = acc[v];
-        }
-        __syncthreads();
-        // the twelve block updates u = 4 ri + j (row block i = ri, skipping kb);
-        // with a next step, wave 0 takes the next pivot block (u0) and the other
-        // eleven go to waves 1-3 in turn, else three to each wave
-        const int nb = kb + 1, u0 = 5 * kb + 1;
-        auto update = [&](int u) {
-            const int ri = u >> 2, j = u & 3, i = ri < kb ? ri : ri + 1;
-            T *Mij = M + 16 * i * LDT + 16 * j;
-            const T *Ci = cur + ri * CS;
-            const bool piv = j == kb;
-            const typename mfma<T>::acc_t acc = mm16<T>(Ci, TMP_LD, piv ? P : M + 16 * kb * LDT + 16 * j, LDT);
-            // the next step's column block of row block i (i != nb)
-            T *sv = (nb < 4 && j == nb && i != nb) ? nxt + (i < nb ? i : i - 1) * CS : nullptr;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = mfma<T>::row(lane, v), c = lane & 15;
-                T &e = Mij[r * LDT + c];
-                const T x = piv ? -acc[v] : e - acc[v];
-                e = x;
-                if (sv) sv[r * TMP_LD + c] = x;
-            }
+        const int nb = kb + 1;
+        auto saved = [&](int i) { return cur + (i < kb ? i : i - 1) * CS; };  // C_i
+        auto column = [&](int j) {
+            T *R = block(kb, j);
+            put(R, LDT, mm16<T>(P, LDT, R, LDT));
+            wave_lds_fence();
+#pragma unroll 1
+            for (int i = 0; i < 4; i++)
+                if (i != kb) update(i, j, saved(i), R, LDT, nullptr);
         };
-        if (nb < 4) {
-            if (wave == 0) {
-                update(u0);
-                pivot_block(nb);
-            } else if (act) {
-                for (int k = wave - 1; k < 11; k += 3) update(k < u0 ? k : k + 1);
-                if (wave == 3) {
-                    // row block kb of the next column blocks: R_nb, final since the products above
-                    const T *src = M + 16 * kb * LDT + 16 * nb;
-                    T *dst = nxt + kb * CS;
-                    for (int t = lane; t < 256; t += 64) dst[(t >> 4) * TMP_LD + (t & 15)] = src[(t >> 4) * LDT + (t & 15)];
+        auto pivot_column = [&] {
+#pragma unroll 1
+            for (int i = 0; i < 4; i++)
+                if (i != kb) {
+                    typename mfma<T>::acc_t acc = mm16<T>(saved(i), TMP_LD, P, LDT);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[e] = -acc[e];
+                    put(block(i, kb), LDT, acc);
                 }
-            }
+        };
+        if (nb == 4) {
+            if (wave < 3) column(wave);
+            else if (act) pivot_column();
+        } else if (wave == 0) {
+            T *R = nxt + kb * CS;
+            put(R, TMP_LD, mm16<T>(P, LDT, block(kb, nb), LDT));
+            wave_lds_fence();
+            update(nb, nb, saved(nb), R, TMP_LD, nullptr);
+            wave_lds_fence();
+            pivot_block(nb);
+        } else if (wave < 3) {
+            column((kb + 1 + wave) & 3);
         } else if (act) {
-            for (int u = wave; u < 12; u += 4) update(u);
+            T *R = tmp + 2 * CB;
+            put(R, TMP_LD, mm16<T>(P, LDT, block(kb, nb), LDT));
+            wave_lds_fence();
+            for (int i = 0; i < 4; i++)
+                if (i != kb && i != nb) update(i, nb, saved(i), R, TMP_LD, nxt + (i < nb ? i : i - 1) * CS);
+            pivot_column();
         }
         __syncthreads();
     }
