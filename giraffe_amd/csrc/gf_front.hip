@@ -13,7 +13,8 @@
 //             the two in elimination order holds it).  Every entry is written by
 //             one thread, in a fixed order: no atomics, bit-reproducible.
 //             The workgroup of each front's first diagonal block also inverts it
-//             (E_0).
+//             (E_0).  Only the tiles of the own rows and columns are written: step 0
+//             forms the others itself.
 //   factor    the block LU of the band solver on each front, restricted to its
 //             kb own block columns, over all fronts of the level at once:
 //             launch p = 0 .. kb - 1 updates A(i, j) -= A(i, p) (E_p A'(p, j))
@@ -36,6 +37,7 @@
 #include "gf_tile.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -135,7 +137,7 @@ __global__ __launch_bounds__(ASM_T, 6) void front_assemble_kernel(FrontTab t, in
     }
     if (it[3] == 0) return;
     // the front's first diagonal block (already in LDS): E_0
-    inverse64<T>(sm.P, sm.tmp, sm.aux, flag);
+    inverse64<T>(sm.P, sm.tmp, sm.aux, flag, min(NB, (F.k + 15) & ~15) >> 4);
     T *E = Eb + F.E;
     for (int q = threadIdx.x; q < NB * NB; q += ASM_T) E[q] = sm.P[(q / NB) * LDT + q % NB];
 }
@@ -155,52 +157,68 @@ template <typename T> struct FStepSmem {
     T aux[4 + NB];
 };
 
-// acc += X(:, k0 .. k0+31) * CT^T, X [i][k] (stride LDT), CT [j][k - k0] (stride SA_LD)
-template <typename T> __device__ __forceinline__ void mm_xc(Acc<T> &acc, const T *X, const T *CT, int k0)
+// acc += X(:, k0 .. k0+31) * CT^T, X [i][k] (stride LDT), CT [j][k - k0] (stride
+// SA_LD); only k < ka and rows < ka (a multiple of 16) take part.
+template <typename T> __device__ __forceinline__ void mm_xc(Acc<T> &acc, const T *X, const T *CT, int k0, int ka)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wr = acc_row(wave), wc = acc_col(wave);
-#pragma unroll 2
-    for (int kk = 0; kk < KT; kk += 4) {
-        T av[2], bv[2];
+    if (wr >= ka) return;
 #pragma unroll
-        for (int x = 0; x < 2; x++) av[x] = X[(wr + 16 * x + (lane & 15)) * LDT + k0 + kk + (lane >> 4)];
+    for (int k16 = 0; k16 < KT; k16 += 16) {
+        if (k0 + k16 >= ka) return;
 #pragma unroll
-        for (int y = 0; y < 2; y++) bv[y] = CT[(wc + 16 * y + (lane & 15)) * SA_LD + kk + (lane >> 4)];
+        for (int kk = k16; kk < k16 + 16; kk += 4) {
+            T av[2], bv[2];
 #pragma unroll
-        for (int x = 0; x < 2; x++)
+            for (int x = 0; x < 2; x++) av[x] = X[(wr + 16 * x + (lane & 15)) * LDT + k0 + kk + (lane >> 4)];
 #pragma unroll
-            for (int y = 0; y < 2; y++) acc.a[x][y] = mfma<T>::run(av[x], bv[y], acc.a[x][y]);
+            for (int y = 0; y < 2; y++) bv[y] = CT[(wc + 16 * y + (lane & 15)) * SA_LD + kk + (lane >> 4)];
+#pragma unroll
+            for (int x = 0; x < 2; x++)
+#pragma unroll
+                for (int y = 0; y < 2; y++) acc.a[x][y] = mfma<T>::run(av[x], bv[y], acc.a[x][y]);
+        }
     }
 }
-// acc += C * XT(:, k0 .. k0+31)^T, C [i][k - k0] (stride SA_LD), XT [j][k] (stride LDT)
-template <typename T> __device__ __forceinline__ void mm_cx(Acc<T> &acc, const T *C, const T *XT, int k0)
+// acc += C * XT(:, k0 .. k0+31)^T, C [i][k - k0] (stride SA_LD), XT [j][k] (stride
+// LDT); only k < ka.
+template <typename T> __device__ __forceinline__ void mm_cx(Acc<T> &acc, const T *C, const T *XT, int k0, int ka)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wr = acc_row(wave), wc = acc_col(wave);
-#pragma unroll 2
-    for (int kk = 0; kk < KT; kk += 4) {
-        T av[2], bv[2];
 #pragma unroll
-        for (int x = 0; x < 2; x++) av[x] = C[(wr + 16 * x + (lane & 15)) * SA_LD + kk + (lane >> 4)];
+    for (int k16 = 0; k16 < KT; k16 += 16) {
+        if (k0 + k16 >= ka) return;
 #pragma unroll
-        for (int y = 0; y < 2; y++) bv[y] = XT[(wc + 16 * y + (lane & 15)) * LDT + k0 + kk + (lane >> 4)];
+        for (int kk = k16; kk < k16 + 16; kk += 4) {
+            T av[2], bv[2];
 #pragma unroll
-        for (int x = 0; x < 2; x++)
+            for (int x = 0; x < 2; x++) av[x] = C[(wr + 16 * x + (lane & 15)) * SA_LD + kk + (lane >> 4)];
 #pragma unroll
-            for (int y = 0; y < 2; y++) acc.a[x][y] = mfma<T>::run(av[x], bv[y], acc.a[x][y]);
+            for (int y = 0; y < 2; y++) bv[y] = XT[(wc + 16 * y + (lane & 15)) * LDT + k0 + kk + (lane >> 4)];
+#pragma unroll
+            for (int x = 0; x < 2; x++)
+#pragma unroll
+                for (int y = 0; y < 2; y++) acc.a[x][y] = mfma<T>::run(av[x], bv[y], acc.a[x][y]);
+        }
     }
 }
 // A 32 x 64 row chunk (rows r0 .. r0+31 of a row-major tile at src, stride ld) into
 // registers (thread t holds t + 256 r: row (t + 256 r) / 64, column t % 64), and
 // into C transposed (C [column][row]).
-template <typename T> __device__ __forceinline__ void rowchunk_load(T (&v)[8], const T *src, size_t ld, int r0)
+// (Here and below a thread's offset into the tile is one 32-bit register, in
+// bytes, and its rows' steps go to the scalar base: per-thread addresses would
+// spill.)
+template <typename T> __device__ __forceinline__ T &at(T *base, unsigned bytes)
 {
+    return *reinterpret_cast<T *>(reinterpret_cast<char *>(const_cast<std::remove_const_t<T> *>(base)) + bytes);
+}
+template <typename T> __device__ __forceinline__ void rowchunk_load(T (&v)[8], const T *src, unsigned ld, int r0)
+{
+    const unsigned o = ((threadIdx.x >> 6) * ld + (threadIdx.x & 63)) * sizeof(T);
 #pragma unroll
-    for (int r = 0; r < 8; r++) {
-        const int t = threadIdx.x + 256 * r;
-        v[r] = src[(size_t)(r0 + (t >> 6)) * ld + (t & 63)];
-    }
+    for (int r = 0; r < 8; r++) v[r] = at(src + (size_t)((r0 + 4 * r) * ld), o);
 }
 template <typename T> __device__ __forceinline__ void rowchunk_put_t(T *C, const T (&v)[8])
 {
@@ -212,13 +230,11 @@ template <typename T> __device__ __forceinline__ void rowchunk_put_t(T *C, const
 }
 // A 64 x 32 column chunk (columns c0 .. c0+31) into registers (thread t holds
 // t + 256 r: row (t + 256 r) / 32, column t % 32), and into C as it is.
-template <typename T> __device__ __forceinline__ void colchunk_load(T (&v)[8], const T *src, size_t ld, int c0)
+template <typename T> __device__ __forceinline__ void colchunk_load(T (&v)[8], const T *src, unsigned ld, int c0)
 {
+    const unsigned o = ((threadIdx.x >> 5) * ld + (threadIdx.x & 31)) * sizeof(T);
 #pragma unroll
-    for (int r = 0; r < 8; r++) {
-        const int t = threadIdx.x + 256 * r;
-        v[r] = src[(size_t)(t >> 5) * ld + c0 + (t & 31)];
-    }
+    for (int r = 0; r < 8; r++) v[r] = at(src + (size_t)(8 * r * ld) + c0, o);
 }
 template <typename T> __device__ __forceinline__ void colchunk_put(T *C, const T (&v)[8])
 {
@@ -229,11 +245,67 @@ template <typename T> __device__ __forceinline__ void colchunk_put(T *C, const T
     }
 }
 
+// The tile element of result item (x, y, v) of a thread: tile + acc_at(x, y, v, ld)
+// at byte offset acc_off(ld).
+template <typename T> __device__ __forceinline__ unsigned acc_off(unsigned ld)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    return ((acc_row(wave) + mfma<T>::row(lane, 0)) * ld + acc_col(wave) + (lane & 15)) * sizeof(T);
+}
+template <typename T> __device__ __forceinline__ size_t acc_at(int x, int y, int v, unsigned ld)
+{
+    return (size_t)((16 * x + mfma<T>::row(0, v)) * ld) + 16 * y;
+}
+
+// Rows (a multiple of 16) of own block p that hold DOFs: the rest of the last
+// block is identity padding, its rows and columns elsewhere zero.
+__device__ __forceinline__ int live_rows(const gf_front_dev &F, int p) { return min(NB, (F.k - NB * p + 15) & ~15); }
+
+// A child's Schur complement entries of a tile at a thread's result positions:
+// first the positions in the child's update rows, then, behind a product, the
+// entries.
+template <typename T> struct ChildTile {
+    int a[2][4], b[2];
+    __device__ __forceinline__ void positions(const FrontTab &t, int c, int R0, int C0)
+    {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const int *im = t.inv + t.child_inv[c];
+#pragma unroll
+        for (int y = 0; y < 2; y++) b[y] = im[C0 + acc_col(wave) + 16 * y + (lane & 15)];
+#pragma unroll
+        for (int x = 0; x < 2; x++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) a[x][v] = im[R0 + acc_row(wave) + 16 * x + mfma<T>::row(lane, v)];
+    }
+    __device__ __forceinline__ void entries(const FrontTab &t, int c, const T *Fb, T (&u)[2][2][4])
+    {
+        const gf_front_dev C = t.fr[t.child[c]];
+        const T *U = Fb + C.F + (size_t)(NB * C.kb) * C.mp + NB * C.kb;
+        acc_each<T>([&](int x, int y, int v, int, int) {
+            u[x][y][v] = T(0);
+            if (a[x][v] >= 0 && b[y] >= 0)
+                u[x][y][v] = at(U, ((unsigned)a[x][v] * (unsigned)C.mp + (unsigned)b[y]) * (unsigned)sizeof(T));
+        });
+    }
+};
+
 // Launch p >= 0 of a level's factorisation (the band step on every front of the
-// level; see the file header).  Item kinds: 0 diagonal, 1 update, 2 conversion.
-// Each product runs in two 32-deep chunks; all of a workgroup's loads are issued
-// before the first product.
-template <typename T>
+// level; see the file header).  Items (front, tile row, tile column, kind | rows
+// << 8), kinds: 0 diagonal, 1 update, 2 conversion.  Each product runs in two
+// 32-deep chunks; all of a workgroup's loads are issued before the first product.
+// An update item covers `rows` tiles of one column: W = E_p A'(p, j) is formed
+// once for them.  One tile is two products of 64^3, of which W is half; launches
+// of more tiles than the device holds at once are bound by those products (45 %
+// of the MFMA rate at one tile an item), so the plan gives them items of several
+// rows while the items still make three rounds (fewer leave the last round
+// empty: 3,584 items of one tile 82 us, 2,560 of two 89); the others are bound by
+// the chain of one workgroup and take one row an item.
+// Padding: a block's products stop at its live rows (33 DOFs of a mesh line fill
+// half of a block).  Launch 0 takes the old value of a tile outside the own rows
+// and columns straight from the children, summed in their order (GATHER; zero
+// for a leaf): the assembly does not write those tiles.  64 x 64 plate, levels 1
+// to 3: assembly 78, 53, 50 -> 43, 29, 35 us, this launch 58, 51, 58 -> 64, 52, 64.
+template <typename T, bool GATHER>
 __global__ __launch_bounds__(256, 3) void front_step_kernel(FrontTab t, int first, int p, T *Fb, T *Eb, int *flag,
                                                          double *Vb)
 {
@@ -242,84 +314,113 @@ __global__ __launch_bounds__(256, 3) void front_step_kernel(FrontTab t, int firs
     const int *it = t.items + 4 * (size_t)(first + blockIdx.x);
     const int f = it[0];
     if (f < 0) return;
-    const int ti = it[1], tj = it[2], kind = it[3];
+    const int ti = it[1], tj = it[2], rows = it[3] >> 8;
+    const int kind = GATHER ? it[3] & 1 : it[3] & 255;  // (launch 0 converts no row)
     if (kind == 0) __builtin_amdgcn_s_setprio(3);
     const gf_front_dev F = t.fr[f];
     T *A = Fb + F.F;
-    const size_t ld = (size_t)F.mp;
+    const unsigned ld = F.mp, ao = acc_off<T>(ld);
     T *Ef = Eb + F.E;
     const int tid = threadIdx.x;
-    const int R0 = ti * NB, C0 = tj * NB;
+    const int C0 = tj * NB;
     // with the right-hand side in the front vector (Vb): the first conversion tile of
     // row p - 1 converts its block, y = E_{p-1} b_{p-1}; the first update tile of row
     // i subtracts L(i, p) y_p, y_p = E_p b_p, from block i (each block written by one
     // workgroup; b_p itself is final and unconverted during launch p)
     const bool rhs_row = Vb && tj == (kind == 2 ? p : p + 1);
-    double *vrow = Vb ? Vb + F.V + (size_t)R0 : nullptr;
     // product 1: W = E_q A'(q, j), q = p (update, diagonal) or p - 1 (conversion)
-    const int q = kind == 2 ? ti : p;
+    const int q = kind == 2 ? ti : p, ka = live_rows(F, q);
     const T *E = Ef + (size_t)q * NB * NB;
-    const T *Aq = A + (size_t)(q * NB) * ld + C0;  // A'(q, j)
+    const T *Aq = A + (size_t)(q * NB * ld) + C0;  // A'(q, j)
     T e[16], a0[8], a1[8];
-    tile_load(e, [&](int i, int k) { return E[i * NB + k]; });
+#pragma unroll
+    for (int r = 0; r < 16; r++) e[r] = at(E + 256 * r, tid * (unsigned)sizeof(T));
     rowchunk_load(a0, Aq, ld, 0);
     rowchunk_load(a1, Aq, ld, KT);
-    if (rhs_row && tid < NB) rv[0][tid] = kind == 2 ? vrow[tid] : Vb[F.V + (size_t)(p * NB) + tid];
+    if (rhs_row && tid < NB) rv[0][tid] = Vb[F.V + (size_t)(q * NB) + tid];
     tile_put(sm.X, LDT, e);
     rowchunk_put_t(sm.C, a0);
     __syncthreads();
     T l0[8], l1[8], old[2][2][4];
-    const T *Lp = A + (size_t)R0 * ld + p * NB;  // L(i, p)
-    if (kind != 2) colchunk_load(l0, Lp, ld, 0);
+    const T *Lp = A + (size_t)(ti * NB * ld) + p * NB;  // L(i, p)
+    colchunk_load(l0, Lp, ld, 0);  // (a conversion item does not use it)
     if (rhs_row && tid < NB) {
         double yv = 0.0;
         for (int c = 0; c < NB; c++) yv += (double)sm.X[tid * LDT + c] * rv[0][c];
-        if (kind == 2) vrow[tid] = yv;
+        if (kind == 2) Vb[F.V + (size_t)(q * NB) + tid] = yv;
         else rv[1][tid] = yv;  // y_p
     }
+    auto tile = [&](int i0) { return A + (size_t)(i0 * NB * ld) + C0; };
     Acc<T> w;
     w.zero();
-    mm_xc<T>(w, sm.X, sm.C, 0);
-    __syncthreads();
-    rowchunk_put_t(sm.C, a1);
-    __syncthreads();
-    if (kind != 2) {
-        // behind the second half of product 1
-        colchunk_load(l1, Lp, ld, KT);
-        acc_each<T>([&](int x, int y, int v, int i, int j) { old[x][y][v] = A[(R0 + i) * ld + C0 + j]; });
+    mm_xc<T>(w, sm.X, sm.C, 0, ka);
+    if (ka > KT) {
+        __syncthreads();
+        rowchunk_put_t(sm.C, a1);
+        __syncthreads();
     }
-    mm_xc<T>(w, sm.X, sm.C, KT);
+    colchunk_load(l1, Lp, ld, KT);  // behind the second half of product 1
+    if (ka > KT) mm_xc<T>(w, sm.X, sm.C, KT, ka);
     if (kind == 2) {
-        acc_each<T>([&](int x, int y, int v, int i, int j) { A[(R0 + i) * ld + C0 + j] = w.a[x][y][v]; });
+        acc_each<T>([&](int x, int y, int v, int, int) { at(tile(ti) + acc_at<T>(x, y, v, ld), ao) = w.a[x][y][v]; });
         return;
     }
     __syncthreads();
     // product 2: old - L(i, p) W, W kept transposed in X
     acc_each<T>([&](int x, int y, int v, int i, int j) { sm.X[j * LDT + i] = w.a[x][y][v]; });
-    colchunk_put(sm.C, l0);
-    __syncthreads();
-    double s = 0.0;
-    if (rhs_row && tid < NB)
-        for (int c = 0; c < KT; c++) s += (double)sm.C[tid * SA_LD + c] * rv[1][c];
     Acc<T> acc;
-    acc.zero();
-    mm_cx<T>(acc, sm.C, sm.X, 0);
-    __syncthreads();
-    colchunk_put(sm.C, l1);
-    __syncthreads();
-    if (rhs_row && tid < NB) {
-        for (int c = 0; c < KT; c++) s += (double)sm.C[tid * SA_LD + c] * rv[1][KT + c];
-        vrow[tid] -= s;  // b_i -= L(i, p) y_p
-    }
-    mm_cx<T>(acc, sm.C, sm.X, KT);
-    if (kind == 1) {
-        acc_each<T>([&](int x, int y, int v, int i, int j) { A[(R0 + i) * ld + C0 + j] = old[x][y][v] - acc.a[x][y][v]; });
-        return;
+    for (int r = 0;; r++) {
+        const int R0 = (ti + r) * NB;
+        colchunk_put(sm.C, l0);
+        __syncthreads();
+        // the old value behind product 2
+        const bool unset = p == 0 && ti + r >= F.kb && tj >= F.kb;
+        ChildTile<T> ct;
+        if (!unset)
+            acc_each<T>([&](int x, int y, int v, int, int) { old[x][y][v] = at(tile(ti + r) + acc_at<T>(x, y, v, ld), ao); });
+        else if (GATHER) ct.positions(t, F.ch0, R0, C0);
+        else acc_each<T>([&](int x, int y, int v, int, int) { old[x][y][v] = T(0); });
+        double s = 0.0;
+        if (rhs_row && tid < NB)
+            for (int c = 0; c < KT; c++) s += (double)sm.C[tid * SA_LD + c] * rv[1][c];
+        acc.zero();
+        mm_cx<T>(acc, sm.C, sm.X, 0, ka);
+        if (ka > KT) {
+            __syncthreads();
+            colchunk_put(sm.C, l1);
+            __syncthreads();
+        }
+        if (GATHER && unset) {
+            ct.entries(t, F.ch0, Fb, old);
+            if (F.ch0 + 1 < F.ch1) ct.positions(t, F.ch0 + 1, R0, C0);
+        }
+        if (ka > KT) {
+            if (rhs_row && tid < NB)
+                for (int c = 0; c < KT; c++) s += (double)sm.C[tid * SA_LD + c] * rv[1][KT + c];
+            mm_cx<T>(acc, sm.C, sm.X, KT, ka);
+        }
+        if (rhs_row && tid < NB) Vb[F.V + R0 + tid] -= s;  // b_i -= L(i, p) y_p
+        if (kind == 0) break;
+        if (GATHER && unset)
+            for (int c = F.ch0 + 1; c < F.ch1; c++) {
+                T u[2][2][4];
+                if (c > F.ch0 + 1) ct.positions(t, c, R0, C0);
+                ct.entries(t, c, Fb, u);
+                acc_each<T>([&](int x, int y, int v, int, int) { old[x][y][v] += u[x][y][v]; });
+            }
+        acc_each<T>([&](int x, int y, int v, int, int) {
+            at(tile(ti + r) + acc_at<T>(x, y, v, ld), ao) = old[x][y][v] - acc.a[x][y][v];
+        });
+        if (r + 1 >= rows) return;
+        Lp += (size_t)(NB * ld);
+        colchunk_load(l0, Lp, ld, 0);
+        colchunk_load(l1, Lp, ld, KT);
+        __syncthreads();
     }
     __syncthreads();
     acc_each<T>([&](int x, int y, int v, int i, int j) { sm.X[i * LDT + j] = old[x][y][v] - acc.a[x][y][v]; });
     __syncthreads();
-    inverse64<T>(sm.X, sm.tmp, sm.aux, flag);  // E_{p+1}
+    inverse64<T>(sm.X, sm.tmp, sm.aux, flag, live_rows(F, ti) >> 4);  // E_{p+1}
     T *En = Ef + (size_t)ti * NB * NB;
     for (int q2 = tid; q2 < NB * NB; q2 += 256) En[q2] = sm.X[(q2 / NB) * LDT + q2 % NB];
 }
@@ -546,8 +647,13 @@ int front_factor_t(const gf_fronts &fp, const double *ab, int ld, int hb, const 
             if (fp.step_count[k] == 0) continue;
             const int p = k - fp.lev_step[l];
             pr = gf_probe_begin(s, GF_KC_FRONT_STEP);
-            hipLaunchKernelGGL(front_step_kernel<T>, dim3(fp.step_count[k]), dim3(256), 0, s, t, fp.step_first[k], p,
-                               F, E, flag, rhs ? V : nullptr);
+            // (leaves are the fronts of level 0)
+            if (p == 0 && l > 0)
+                hipLaunchKernelGGL((front_step_kernel<T, true>), dim3(fp.step_count[k]), dim3(256), 0, s, t,
+                                   fp.step_first[k], p, F, E, flag, rhs ? V : nullptr);
+            else
+                hipLaunchKernelGGL((front_step_kernel<T, false>), dim3(fp.step_count[k]), dim3(256), 0, s, t,
+                                   fp.step_first[k], p, F, E, flag, rhs ? V : nullptr);
             gf_probe_end(s, pr, fp.step_flops[k]);
             launches++;
         }

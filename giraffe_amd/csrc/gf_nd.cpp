@@ -313,21 +313,30 @@ int gf_nd_plan(gf_fronts &fp, const gf_model_desc *d, const std::vector<int> &do
         for (int p = 0; p < fp.lev_kb[l]; p++) {
             std::vector<std::vector<int>> diag(8), rest(8);
             double fl = 0.0;
+            // tile rows of an update item: up to four, as long as the items still fill
+            // the device (three workgroups on each of 256 CUs) three times over
+            long long tiles = 0;
+            for (int f = fp.lev_off[l]; f < fp.lev_off[l + 1]; f++)
+                if (p < fp.fr[f].kb) tiles += (long long)(fp.fr[f].mb - p - 1) * (fp.fr[f].mb - p - 1);
+            const int strip = (int)std::min(4LL, std::max(1LL, tiles / (3 * 768)));
             for (int f = fp.lev_off[l]; f < fp.lev_off[l + 1]; f++) {
                 const gf_front_dev &F = fp.fr[f];
                 const int x0 = f;
                 if (p < F.kb) {
-                    for (int i = p + 1; i < F.mb; i++)
-                        for (int j = p + 1; j < F.mb; j++) {
-                            const bool dg = i == p + 1 && j == p + 1 && p + 1 < F.kb;
-                            auto &q = dg ? diag[(x0 + i) & 7] : rest[(x0 + i) & 7];
-                            q.insert(q.end(), {f, i, j, dg ? 0 : 1});
+                    const bool dg = p + 1 < F.kb;  // a next pivot: its tile is an item of its own
+                    if (dg) diag[(x0 + p + 1) & 7].insert(diag[(x0 + p + 1) & 7].end(), {f, p + 1, p + 1, 0 | 1 << 8});
+                    for (int j = p + 1; j < F.mb; j++)
+                        for (int i0 = p + 1 + (dg && j == p + 1); i0 < F.mb;) {
+                            const int n = std::min(strip, F.mb - i0);
+                            auto &q = rest[(x0 + i0) & 7];
+                            q.insert(q.end(), {f, i0, j, 1 | n << 8});
+                            i0 += n;
                         }
                     const int m = kvec[f] + uvec[f];
                     for (int c = TB * p; c < std::min(TB * (p + 1), kvec[f]); c++) fl += 2.0 * (double)(m - c - 1) * (m - c - 1);
                 }
                 if (p >= 1 && p <= F.kb - 1)
-                    for (int j = p; j < F.mb; j++) rest[(x0 + p - 1) & 7].insert(rest[(x0 + p - 1) & 7].end(), {f, p - 1, j, 2});
+                    for (int j = p; j < F.mb; j++) rest[(x0 + p - 1) & 7].insert(rest[(x0 + p - 1) & 7].end(), {f, p - 1, j, 2 | 1 << 8});
             }
             for (int x = 0; x < 8; x++) diag[x].insert(diag[x].end(), rest[x].begin(), rest[x].end());
             const int first = emit(diag);
@@ -341,13 +350,14 @@ int gf_nd_plan(gf_fronts &fp, const gf_model_desc *d, const std::vector<int> &do
     // assembly tiles and solve row tiles per level
     for (int l = 0; l < nlev; l++) {
         // assembly tiles, the first diagonal block of every front first (kind 1:
-        // assembled and inverted)
+        // assembled and inverted); the tiles outside the own rows and columns are
+        // formed by step 0, which is the first to touch them
         const int a0 = (int)fp.items.size() / 4;
         for (int f = fp.lev_off[l]; f < fp.lev_off[l + 1]; f++) fp.items.insert(fp.items.end(), {f, 0, 0, 1});
         for (int f = fp.lev_off[l]; f < fp.lev_off[l + 1]; f++)
             for (int i = 0; i < fp.fr[f].mb; i++)
                 for (int j = 0; j < fp.fr[f].mb; j++)
-                    if (i || j) fp.items.insert(fp.items.end(), {f, i, j, 0});
+                    if ((i || j) && (i < fp.fr[f].kb || j < fp.fr[f].kb)) fp.items.insert(fp.items.end(), {f, i, j, 0});
         fp.asm_first.push_back(a0);
         fp.asm_count.push_back((int)fp.items.size() / 4 - a0);
         const int u0 = (int)fp.items.size() / 4;

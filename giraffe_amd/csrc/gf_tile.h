@@ -327,8 +327,9 @@ __device__ __forceinline__ void wave_lds_fence()
 // with perturbed pivots is still refined against the FP64 tangent, which
 // decides whether it was good enough.)  tmp: INV_TMP entries; aux: 4 + 64
 // entries.  Runs on the first four wavefronts; those of a larger workgroup only
-// take part in the barriers.
-template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T *aux, int *flag)
+// take part in the barriers.  nk: only the first nk row and column blocks are
+// inverted (the rest is identity, decoupled).
+template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T *aux, int *flag, int nk = 4)
 {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const bool act = tid < 256;
@@ -386,7 +387,7 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
     }
     __syncthreads();
 #pragma unroll 1
-    for (int kb = 0; kb < 4; kb++) {
+    for (int kb = 0; kb < nk; kb++) {
         const T *cur = tmp + (kb & 1) * CB, *P = block(kb, kb);
         T *nxt = tmp + ((kb + 1) & 1) * CB;
         const int nb = kb + 1;
@@ -396,12 +397,12 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
             put(R, LDT, mm16<T>(P, LDT, R, LDT));
             wave_lds_fence();
 #pragma unroll 1
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < nk; i++)
                 if (i != kb) update(i, j, saved(i), R, LDT, nullptr);
         };
         auto pivot_column = [&] {
 #pragma unroll 1
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < nk; i++)
                 if (i != kb) {
                     typename mfma<T>::acc_t acc = mm16<T>(saved(i), TMP_LD, P, LDT);
 #pragma unroll
@@ -409,9 +410,9 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
                     put(block(i, kb), LDT, acc);
                 }
         };
-        if (nb == 4) {
-            if (wave < 3) column(wave);
-            else if (act) pivot_column();
+        if (nb == nk) {
+            if (wave < nb - 1) column(wave);
+            else if (wave == nb - 1) pivot_column();
         } else if (wave == 0) {
             T *R = nxt + kb * CS;
             put(R, TMP_LD, mm16<T>(P, LDT, block(kb, nb), LDT));
@@ -420,12 +421,14 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
             wave_lds_fence();
             pivot_block(nb);
         } else if (wave < 3) {
-            column((kb + 1 + wave) & 3);
+            // the columns other than kb and nb, in cyclic order
+            const int j = (kb + 1 + wave) % nk;
+            if (1 + wave < nk) column(j);
         } else if (act) {
             T *R = tmp + 2 * CB;
             put(R, TMP_LD, mm16<T>(P, LDT, block(kb, nb), LDT));
             wave_lds_fence();
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < nk; i++)
                 if (i != kb && i != nb) update(i, nb, saved(i), R, TMP_LD, nxt + (i < nb ? i : i - 1) * CS);
             pivot_column();
         }
