@@ -531,6 +531,61 @@ __global__ __launch_bounds__(256) void front_fwd_upd_kernel(FrontTab t, int firs
     if ((tid & 3) == 0) Vb[F.V + i] = c - part;
 }
 
+// The backward kernels (one workgroup of four wavefronts a row tile or front)
+// read tiles whole rows at a time: wavefront w takes rows 16 w .. 16 w + 15 in
+// pairs, lane l the columns 2 (l % 32) and the next of row l / 32 of a pair, so a
+// load instruction covers 1 KB in eight lines.  With a quad of lanes a row, each
+// lane 128 contiguous bytes, every instruction touched 64 lines and a tile took
+// four times as long to come through the CU's cache, which is what these few
+// workgroups are bound by: a row of 9 update tiles 15 -> 9.5 us, the 64 x 64
+// plate's root (9 own blocks, 36 tiles) 44 -> 29 us, its leaves 28 -> 22 us.  (Four
+// quad-row groups on more tiles at once made the root 66 us: same bound.)  A lane
+// keeps the partial sums of its eight rows over
+// all tiles; the 32 lanes of a row are summed once at the end.
+template <typename T> struct RowTile {
+    T v[16];
+    __device__ __forceinline__ void load(const T *tile, unsigned ld)
+    {
+        typedef T pair_t __attribute__((ext_vector_type(2)));
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const unsigned o = ((16 * wave + (lane >> 5)) * ld + 2 * (lane & 31)) * sizeof(T);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const pair_t w = *reinterpret_cast<const pair_t *>(&at(tile + (size_t)(2 * k * ld), o));
+            v[2 * k] = w.x;
+            v[2 * k + 1] = w.y;
+        }
+    }
+    // acc[k] += this lane's part of row 2 k + l / 32 times y (LDS, the tile's 64 columns)
+    __device__ __forceinline__ void dot(double (&acc)[8], const double *y) const
+    {
+        const double2 w = *reinterpret_cast<const double2 *>(y + 2 * (threadIdx.x & 31));
+#pragma unroll
+        for (int k = 0; k < 8; k++) acc[k] = fma((double)v[2 * k + 1], w.y, fma((double)v[2 * k], w.x, acc[k]));
+    }
+};
+// Sum of the partials over the 32 lanes of a row; the lane gets that of tile row
+// tile_row() (four lanes share one).
+__device__ __forceinline__ int tile_row()
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    return 16 * wave + 2 * ((lane >> 4 & 1) * 4 + (lane >> 3 & 1) * 2 + (lane >> 2 & 1)) + (lane >> 5);
+}
+__device__ __forceinline__ double tile_sum(double (&acc)[8])
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int n = 4; n >= 1; n >>= 1) {  // halve the rows, xor 16, 8, 4
+        const bool up = lane & (4 * n);
+#pragma unroll
+        for (int k = 0; k < n; k++) {
+            const double give = up ? acc[k] : acc[k + n], keep = up ? acc[k + n] : acc[k];
+            acc[k] = keep + __shfl_xor(give, 4 * n);
+        }
+    }
+    return quad_sum(acc[0]);
+}
+
 // Own row tile p of a front with an update part: z_p = y_p - U(p, update) x_update
 // (x_update gathered from the ancestors' rows of x into LDS, 1024 at a time).
 template <typename T>
@@ -540,10 +595,15 @@ __global__ __launch_bounds__(256) void front_bwd_upd_kernel(FrontTab t, int firs
     __shared__ double xu[KMAX];
     const int *it = t.items + 4 * (size_t)(first + blockIdx.x);
     const gf_front_dev F = t.fr[it[0]];
-    const int p = it[1], tid = threadIdx.x, r = tid >> 2, sg = 16 * (tid & 3);
+    const int p = it[1], tid = threadIdx.x, r = tile_row();
     const int *rows = t.rows + F.rows;
-    const T *U = Fb + F.F + (size_t)(NB * p + r) * F.mp + sg;
-    double part = 0.0;
+    const unsigned ld = F.mp;
+    const T *U = Fb + F.F + (size_t)(NB * p * ld);
+    const bool last = p == F.kb - 1, lead = (tid & 3) == 0;
+    double acc[8] = {}, *z = Vb + F.V + NB * p;
+    RowTile<T> a;
+    a.load(U + NB * F.kb, ld);
+    const double y = lead ? z[r] : 0.0;
     for (int c0 = NB * F.kb; c0 < F.mp; c0 += KMAX) {
         const int cn = min(KMAX, F.mp - c0);
         __syncthreads();
@@ -552,30 +612,29 @@ __global__ __launch_bounds__(256) void front_bwd_upd_kernel(FrontTab t, int firs
             xu[j] = o >= 0 ? x[o] : 0.0;
         }
         __syncthreads();
-        for (int q = 0; q < cn / NB; q++) {
-            T v[16];
-            load16(U + c0 + NB * q, v);
-            part += dot16(v, xu + NB * q + sg);
+        for (int q = 0; q < cn; q += NB) {
+            RowTile<T> b;
+            if (c0 + q + NB < F.mp) b.load(U + c0 + q + NB, ld);
+            a.dot(acc, xu + q);
+            a = b;
         }
-    }
-    part = quad_sum(part);
-    if (p < F.kb - 1) {
-        if ((tid & 3) == 0) Vb[F.V + NB * p + r] -= part;
-        return;
     }
     // the last own block row holds A'(p, .) = D_p U(p, .): subtract E_p (A' x); when
     // the factorisation carried the right-hand side, its block is unconverted too:
     // z_p = E_p (b_p - A' x)
-    T e[16];
-    load16(Eb + F.E + (size_t)p * NB * NB + r * NB + sg, e);
-    __syncthreads();
-    if ((tid & 3) == 0) xu[r] = raw_last ? Vb[F.V + NB * p + r] - part : part;
-    __syncthreads();
-    part = quad_sum(dot16(e, xu + sg));
-    if ((tid & 3) == 0) {
-        if (raw_last) Vb[F.V + NB * p + r] = part;
-        else Vb[F.V + NB * p + r] -= part;
+    if (last) a.load(Eb + F.E + (size_t)(p * NB * NB), NB);
+    const double part = tile_sum(acc);
+    if (!last) {
+        if (lead) z[r] = y - part;
+        return;
     }
+    __syncthreads();
+    if (lead) xu[r] = raw_last ? y - part : part;
+    __syncthreads();
+    double e[8] = {};
+    a.dot(e, xu);
+    const double s = tile_sum(e);
+    if (lead) z[r] = raw_last ? s : y - s;
 }
 
 // Own-block back substitution x_p = z_p - sum_{p < j < kb} U(p, j) x_j, then the
@@ -587,31 +646,39 @@ __global__ __launch_bounds__(256) void front_bwd_own_kernel(FrontTab t, int f0, 
     __shared__ double y[KMAX];
     const int f = f0 + blockIdx.x;
     const gf_front_dev F = t.fr[f];
-    const int kp = NB * F.kb, tid = threadIdx.x, r = tid >> 2, sg = 16 * (tid & 3);
+    const int kp = NB * F.kb, tid = threadIdx.x, r = tile_row();
     const int *rows = t.rows + F.rows;
-    const size_t ld = (size_t)F.mp;
+    const unsigned ld = F.mp;
+    const T *U = Fb + F.F;
+    const bool lead = (tid & 3) == 0;
+    // each row's first tile is loaded before the row it waits for is done
+    RowTile<T> a;
+    if (F.kb > 1) a.load(U + (size_t)(NB * (F.kb - 2) * ld) + NB * (F.kb - 1), ld);
     for (int i = tid; i < kp; i += 256) y[i] = Vb[F.V + i];
     __syncthreads();
     if (raw_last && F.mb == F.kb) {
         // no update part, so no front_bwd_upd_kernel converted the last block: y = E b
-        const int p = F.kb - 1;
-        T e[16];
-        load16(Eb + F.E + (size_t)p * NB * NB + r * NB + sg, e);
-        const double v = quad_sum(dot16(e, y + NB * p + sg));
+        RowTile<T> e;
+        double acc[8] = {};
+        e.load(Eb + F.E + (size_t)((F.kb - 1) * NB * NB), NB);
+        e.dot(acc, y + NB * (F.kb - 1));
+        const double s = tile_sum(acc);
         __syncthreads();
-        if ((tid & 3) == 0) y[NB * p + r] = v;
+        if (lead) y[NB * (F.kb - 1) + r] = s;
         __syncthreads();
     }
     for (int p = F.kb - 2; p >= 0; p--) {
-        const T *U = Fb + F.F + (size_t)(NB * p + r) * ld + sg;
-        double part = 0.0;
+        const T *Up = U + (size_t)(NB * p * ld);
+        double acc[8] = {};
         for (int j = p + 1; j < F.kb; j++) {
-            T v[16];
-            load16(U + NB * j, v);
-            part += dot16(v, y + NB * j + sg);
+            RowTile<T> b;
+            if (j + 1 < F.kb) b.load(Up + NB * (j + 1), ld);
+            else if (p > 0) b.load(Up - (size_t)(NB * ld) + NB * p, ld);
+            a.dot(acc, y + NB * j);
+            a = b;
         }
-        part = quad_sum(part);
-        if ((tid & 3) == 0) y[NB * p + r] -= part;
+        const double s = tile_sum(acc);
+        if (lead) y[NB * p + r] -= s;
         __syncthreads();
     }
     for (int i = tid; i < F.k; i += 256) x[rows[i]] = y[i];
