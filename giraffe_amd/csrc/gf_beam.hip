@@ -5,9 +5,7 @@
 // MountFieldLoading (gravity) :838-878, MountGlobal :1429-1492,
 // SaveLagrange :1494-1506, PreCalc :501-692.
 //
-// Work split per workgroup of one wavefront (64 lanes) and EPB = 7 elements
-// (a colour of 5,000 elements is 715 workgroups, so every CU holds several and
-// their latencies overlap):
+// Work split per workgroup of EPB = 7 elements:
 //   phase 1 -- one lane per (element, Gauss point): Rodrigues kinematics,
 //              back-rotated strains, stresses and the 9x9 operator
 //              M = B^T D B + G (block-sparse: 7 non-zero 3x3 blocks) plus
@@ -18,6 +16,12 @@
 //              global frame (T3^T S T3) and added into the matrix;
 //   phase 3 -- one lane per (element, node): internal force minus self-weight
 //              subtracted from the residual r = f_ext - f_int.
+// The kernel takes a whole SIMD's registers a wavefront.  While a launch's
+// workgroups all fit the device with two of them (512), a second wavefront runs
+// phases 1 and 3 beside the first's phase 2, whose data, old matrix entries
+// included, is read during phase 1: such a launch is one chain of latencies,
+// 14.2 us with the three phases in a row and 11.7 us so.  Beyond, one wavefront
+// takes the phases in a row (715 workgroups: 23 us, two wavefronts each 27).
 // Elements are sorted by colour (no two elements of a colour share a node),
 // so one launch per colour scatters without atomics and deterministically.
 #include "gf_internal.h"
@@ -26,7 +30,7 @@
 namespace {
 
 constexpr int EPB = 7;       // elements per workgroup
-constexpr int WG = 64;
+constexpr int WG = 64;      // threads of a wavefront; two of them in the split form
 constexpr int LDS_GP = 73;   // 7 blocks * 9 + 9 (B^T sigma) + the Gauss point's mass per length
 
 struct BeamGP {
@@ -90,8 +94,8 @@ __device__ __forceinline__ void gather_disp(const double *__restrict__ disp, con
 // buoy (null: none): Pipe_1 buoyant mass per length, applied at Gauss points
 // below the ocean surface through `surf` (a point of it), with the converged
 // coordinates `copy`.
-template <int MODE>
-__global__ __launch_bounds__(WG) void beam_assemble_kernel(
+template <int MODE, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 2 * WG : WG) void beam_assemble_kernel(
     int e0, int e1, size_t ld, const int *__restrict__ conn, const double *__restrict__ cst,
     const double *__restrict__ gps, const double *__restrict__ disp, const int *__restrict__ dof,
     gf_gmat gm, double *__restrict__ r, const double *__restrict__ lfp, double gx, double gy, double gz,
@@ -99,13 +103,61 @@ __global__ __launch_bounds__(WG) void beam_assemble_kernel(
     const double *__restrict__ copy, double sx, double sy, double sz)
 {
     __shared__ double sm[EPB * 2 * LDS_GP];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x & 63;
+    const bool w0 = !SPLIT || threadIdx.x < 64, w1 = !SPLIT || threadIdx.x >= 64;  // phase 2; phases 1 and 3
     const int ebase = e0 + blockIdx.x * EPB;
     // gravity ramp factor, device-resident so a captured Newton step reads the current one
     const double lf = lfp ? *lfp : 0.0;
 
+    // ---- phase 2's own data -------------------------------------------------
+    const int le2 = tid / 9, ab2 = tid - 9 * le2, a2 = ab2 / 3, b2 = ab2 - 3 * a2, e2 = ebase + le2;
+    const bool pair = w0 && tid < 9 * EPB && e2 < e1;
+    double w = 0.0, Na2[2], Nb2[2], dNa2[2], dNb2[2];
+    m3<double> T2;
+    double old36[36], *base36 = gm.layout == GM_BTD ? gm.A : gm.ab;
+    unsigned off36[36];  // entries from base36 (both layouts hold fewer than 2^32)
+    bool okr[6], okc[6];
+    auto fetch = [&] {
+        if (!pair) return;
+        w = cst[BC_JAC * ld + e2];
+#pragma unroll
+        for (int gp = 0; gp < 2; gp++) {
+            Na2[gp] = cst[(BC_N + 3 * gp + a2) * ld + e2];
+            Nb2[gp] = cst[(BC_N + 3 * gp + b2) * ld + e2];
+            dNa2[gp] = cst[(BC_DN + 3 * gp + a2) * ld + e2];
+            dNb2[gp] = cst[(BC_DN + 3 * gp + b2) * ld + e2];
+        }
+#pragma unroll
+        for (int i = 0; i < 9; i++) T2.a[i] = cst[(BC_T3 + i) * ld + e2];
+        if (MODE == 0) {
+            const int na = conn[a2 * ld + e2], nbn = conn[b2 * ld + e2];
+            int rr[6], cc[6];
+#pragma unroll
+            for (int k = 0; k < 6; k++) {
+                rr[k] = dof[6 * na + k];
+                cc[k] = dof[6 * nbn + k];
+                okr[k] = rr[k] >= 0;
+                okc[k] = cc[k] >= 0;
+            }
+            int R36[36], C36[36];
+#pragma unroll
+            for (int k = 0; k < 36; k++) {
+                R36[k] = rr[k / 6];
+                C36[k] = cc[k % 6];
+            }
+            double *p36[36];
+            gm_addr_n<36>(gm, R36, C36, p36);
+#pragma unroll
+            for (int k = 0; k < 36; k++) {
+                off36[k] = (unsigned)(p36[k] - base36);
+                old36[k] = base36[off36[k]];
+            }
+        }
+    };
+    if (SPLIT) fetch();
+
     // ---- phase 1: per (element, Gauss point) -------------------------------
-    if (tid < 2 * EPB) {
+    if (w1 && tid < 2 * EPB) {
         int le = tid >> 1, gp = tid & 1;
         int e = ebase + le;
         if (e < e1) {
@@ -197,74 +249,48 @@ __global__ __launch_bounds__(WG) void beam_assemble_kernel(
     __syncthreads();
 
     // ---- phase 2: per (element, node pair) --------------------------------
-    if (tid < 9 * EPB) {
-        int le = tid / 9, ab = tid - 9 * (tid / 9);
-        int a = ab / 3, b = ab - 3 * (ab / 3);
-        int e = ebase + le;
-        if (e < e1) {
-            double w = cst[BC_JAC * ld + e];
-            m3<double> uu, ua, au, aa;
+    if (!SPLIT) fetch();
+    if (pair) {
+        m3<double> uu, ua, au, aa;
 #pragma unroll
-            for (int i = 0; i < 9; i++) uu.a[i] = ua.a[i] = au.a[i] = aa.a[i] = 0.0;
+        for (int i = 0; i < 9; i++) uu.a[i] = ua.a[i] = au.a[i] = aa.a[i] = 0.0;
 #pragma unroll
-            for (int gp = 0; gp < 2; gp++) {
-                const double *o = sm + (le * 2 + gp) * LDS_GP;
-                double Na = cst[(BC_N + 3 * gp + a) * ld + e], Nb = cst[(BC_N + 3 * gp + b) * ld + e];
-                double dNa = cst[(BC_DN + 3 * gp + a) * ld + e], dNb = cst[(BC_DN + 3 * gp + b) * ld + e];
-                double c00 = w * dNa * dNb, c02 = w * dNa * Nb, c20 = w * Na * dNb, c22 = w * Na * Nb;
+        for (int gp = 0; gp < 2; gp++) {
+            const double *o = sm + (le2 * 2 + gp) * LDS_GP;
+            const double Na = Na2[gp], Nb = Nb2[gp], dNa = dNa2[gp], dNb = dNb2[gp];
+            double c00 = w * dNa * dNb, c02 = w * dNa * Nb, c20 = w * Na * dNb, c22 = w * Na * Nb;
 #pragma unroll
-                for (int i = 0; i < 9; i++) {
-                    uu.a[i] += c00 * o[i];
-                    ua.a[i] += c02 * o[9 + i];
-                    au.a[i] += c20 * o[36 + i];
-                    aa.a[i] += c00 * o[18 + i] + c02 * o[27 + i] + c20 * o[45 + i] + c22 * o[54 + i];
-                }
+            for (int i = 0; i < 9; i++) {
+                uu.a[i] += c00 * o[i];
+                ua.a[i] += c02 * o[9 + i];
+                au.a[i] += c20 * o[36 + i];
+                aa.a[i] += c00 * o[18 + i] + c02 * o[27 + i] + c20 * o[45 + i] + c22 * o[54 + i];
             }
-            m3<double> T3;
+        }
+        m3<double> blk[4];
+        blk[0] = mtm3(T2, mm3(uu, T2));
+        blk[1] = mtm3(T2, mm3(ua, T2));
+        blk[2] = mtm3(T2, mm3(au, T2));
+        blk[3] = mtm3(T2, mm3(aa, T2));
+        if (MODE == 0) {
 #pragma unroll
-            for (int i = 0; i < 9; i++) T3.a[i] = cst[(BC_T3 + i) * ld + e];
-            m3<double> blk[4];
-            blk[0] = mtm3(T3, mm3(uu, T3));
-            blk[1] = mtm3(T3, mm3(ua, T3));
-            blk[2] = mtm3(T3, mm3(au, T3));
-            blk[3] = mtm3(T3, mm3(aa, T3));
-            if (MODE == 0) {
-                int na = conn[a * ld + e], nbn = conn[b * ld + e];
-                int rr[6], cc[6];
+            for (int i = 0; i < 6; i++)
 #pragma unroll
-                for (int k = 0; k < 6; k++) { rr[k] = dof[6 * na + k]; cc[k] = dof[6 * nbn + k]; }
-                int R36[36], C36[36];
-                double V36[36];
+                for (int j = 0; j < 6; j++)
+                    if (okr[i] && okc[j])
+                        base36[off36[6 * i + j]] = old36[6 * i + j] + blk[2 * (i / 3) + j / 3].a[3 * (i % 3) + j % 3];
+        } else {
+            double *Ke = Kout + (size_t)e2 * 324;
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    int ro = (q >> 1) * 3, co = (q & 1) * 3;
+            for (int i = 0; i < 6; i++)
 #pragma unroll
-                    for (int i = 0; i < 3; i++)
-#pragma unroll
-                        for (int j = 0; j < 3; j++) {
-                            const int k = 9 * q + 3 * i + j;
-                            R36[k] = rr[ro + i];
-                            C36[k] = cc[co + j];
-                            V36[k] = blk[q].a[3 * i + j];
-                        }
-                }
-                gm_add_n<36>(gm, R36, C36, V36);
-            } else {
-                double *Ke = Kout + (size_t)e * 324;
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    int ro = (q >> 1) * 3, co = (q & 1) * 3;
-#pragma unroll
-                    for (int i = 0; i < 3; i++)
-#pragma unroll
-                        for (int j = 0; j < 3; j++) Ke[(6 * a + ro + i) * 18 + 6 * b + co + j] = blk[q].a[3 * i + j];
-                }
-            }
+                for (int j = 0; j < 6; j++)
+                    Ke[(6 * a2 + i) * 18 + 6 * b2 + j] = blk[2 * (i / 3) + j / 3].a[3 * (i % 3) + j % 3];
         }
     }
 
     // ---- phase 3: per (element, node): internal force - self-weight --------
-    if (tid < 3 * EPB) {
+    if (w1 && tid < 3 * EPB) {
         int le = tid / 3, a = tid - 3 * (tid / 3);
         int e = ebase + le;
         if (e < e1) {
@@ -446,11 +472,15 @@ int gf_beam_assemble(gf_model *m, const double *lfp)
         launches++;
         int grid = (e1 - e0 + EPB - 1) / EPB;
         const int pr = gf_probe_begin(m->stream, GF_KC_BEAM_ASSEMBLE);
-        hipLaunchKernelGGL(beam_assemble_kernel<0>, dim3(grid), dim3(WG), 0, m->stream, e0, e1, ld, m->d_bconn,
-                           m->d_bconst, m->d_bgp, m->d_disp, m->d_dof, gf_model_gmat(m), m->d_r, lfp, m->gravity[0],
-                           m->gravity[1], m->gravity[2], (double *)nullptr, (double *)nullptr,
-                           (const double *)m->d_bbuoy, (const double *)m->d_copy, m->ocean_surface[0],
-                           m->ocean_surface[1], m->ocean_surface[2]);
+        auto launch = [&](auto kernel, int threads) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, m->stream, e0, e1, ld, m->d_bconn, m->d_bconst,
+                               m->d_bgp, m->d_disp, m->d_dof, gf_model_gmat(m), m->d_r, lfp, m->gravity[0],
+                               m->gravity[1], m->gravity[2], (double *)nullptr, (double *)nullptr,
+                               (const double *)m->d_bbuoy, (const double *)m->d_copy, m->ocean_surface[0],
+                               m->ocean_surface[1], m->ocean_surface[2]);
+        };
+        if (grid <= 512) launch(beam_assemble_kernel<0, true>, 2 * WG);
+        else launch(beam_assemble_kernel<0, false>, WG);
         gf_probe_end(m->stream, pr, e1 - e0);
     }
     GF_HIP(hipGetLastError());
@@ -509,7 +539,7 @@ int gf_beam_eval_device(int count, const double *x, const double *cs, const doub
     GF_HIP(hipMemcpyAsync(d_disp, disp.data(), sizeof(double) * disp.size(), hipMemcpyHostToDevice, s));
     int grid = (count + EPB - 1) / EPB;
     gf_gmat none = {};
-    hipLaunchKernelGGL(beam_assemble_kernel<1>, dim3(grid), dim3(WG), 0, s, 0, count, ld, d_conn, d_cst, d_gps,
+    hipLaunchKernelGGL((beam_assemble_kernel<1, false>), dim3(grid), dim3(WG), 0, s, 0, count, ld, d_conn, d_cst, d_gps,
                        d_disp, (const int *)nullptr, none, (double *)nullptr, (const double *)nullptr, 0.0, 0.0, 0.0, d_K,
                        d_f,
                        (const double *)nullptr, (const double *)nullptr, 0.0, 0.0, 0.0);

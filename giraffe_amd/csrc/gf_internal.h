@@ -396,6 +396,7 @@ inline void gf_probe_end(hipStream_t s, int slot, double units, int count = 1)
 // step (read by the assembly kernels, so a captured Newton step replays with
 // the step's values)
 enum { GF_SCAL_INC = 0, GF_SCAL_FLAG = 8, GF_SCAL_RES = 16, GF_SCAL_REF = 24, GF_SCAL_TIME = 28, GF_SCAL_LF = 29,
+       GF_SCAL_TICKET = 30,
        GF_SCAL_N = 32 };
 
 struct gf_model {
@@ -510,6 +511,7 @@ struct gf_model {
     int npad = 0;                   // padded system size
     double *d_scal = nullptr;       // small reduction results
     double *h_scal = nullptr;       // pinned mirror
+    bool scal_clear = false;        // d_scal[0..GF_SCAL_FLAG] is zero once the stream is there
     int *d_flag = nullptr;          // solver failure flag
     bool factored = false;
 
@@ -563,6 +565,10 @@ gf_gmat gf_model_gmat(const gf_model *m);
 int gf_nodal_loads(gf_model *m, const double *tp);
 int gf_scan_residual(gf_model *m);
 int gf_update_disp(gf_model *m, bool zero_norms);
+int gf_update_clear(gf_model *m);
+// The tangent's storage and, as clear3 takes it, the unit diagonal of its padding rows.
+void gf_assemble_clear_ranges(const gf_model *m, double *&tan, size_t &ntan, size_t &dfirst, size_t &dstride,
+                              size_t &dcount);
 int gf_node_commit(gf_model *m);
 
 int gf_btd_alloc(gf_btd &b, int m, int nblk, int elem_size);
@@ -577,7 +583,7 @@ int gf_btd_factor_solve(const gf_btd &b, hipStream_t s, int *d_flag, const doubl
 
 // Asynchronous halves of gf_assemble and gf_solve + gf_update: *_enqueue puts the
 // work on the model's stream, *_result reads the norms once the stream passed it.
-int gf_assemble_enqueue(gf_model *m, bool copy_norms);
+int gf_assemble_enqueue(gf_model *m, bool cleared);
 int gf_assemble_result(gf_model *m, double *res_out);
 int gf_solve_update_enqueue(gf_model *m, bool then_assemble);
 int gf_solve_update_result(gf_model *m, int *info_fail, double *inc_out);

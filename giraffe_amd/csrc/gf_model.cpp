@@ -784,9 +784,10 @@ static int create(const gf_model_desc *d, const gf_options *opt, gf_model *m)
     }
     if (m->precision == GF_PREC_MIXED) GF_TRY(gf_mixed_alloc(m));
     // scalar block (doubles): [0..4] increment norms, [8] solver failure flag
-    // (int), [16..18] residual norms, [24..25] refinement norms; one copy of
-    // [0..18] returns a whole Newton iteration's results
+    // (int), [16..18] residual norms, [24..25] refinement norms; [0..18] are a whole
+    // Newton iteration's results
     GF_TRY(dalloc(&m->d_scal, GF_SCAL_N));
+    GF_TRY(gf_launch_fill(m->stream, m->d_scal, GF_SCAL_N, 0.0));
     m->d_flag = (int *)(m->d_scal + GF_SCAL_FLAG);
     GF_TRY(gf_pinned_alloc((void **)&m->h_scal, GF_SCAL_N * sizeof(double)));
     for (int i = 0; i < 2 * GF_NPHASE; i++) GF_HIP(hipEventCreate(&m->ev[i]));
@@ -1061,33 +1062,46 @@ extern "C" int gf_set_solution_window(gf_model *m, double start, double end)
     return set_step_scalars(m);
 }
 
-// Enqueues Clear + MountLocal/ElementLoads/Loads + MountGlobal and the residual
-// max-norm scan (norms at d_scal[GF_SCAL_RES..+2]); copy_norms: also copy them
-// to h_scal (a caller that copies the scalar block itself passes false).
-int gf_assemble_enqueue(gf_model *m, bool copy_norms)
+void gf_assemble_clear_ranges(const gf_model *m, double *&tan, size_t &ntan, size_t &dfirst, size_t &dstride,
+                              size_t &dcount)
+{
+    // the padding rows [n_free, npad) carry a unit diagonal (all in the last block
+    // row for the block-tridiagonal layout)
+    const size_t nf = (size_t)m->n_free;
+    dcount = (size_t)m->npad - nf;
+    if (m->layout == GM_BTD) {
+        const size_t mb = (size_t)m->btd.m, last = (size_t)m->btd.nblk - 1, i0 = nf - last * mb;
+        tan = (double *)m->btd.A;
+        ntan = 3 * (size_t)m->btd.nblk * m->btd.bsz;
+        dfirst = (size_t)m->btd.nblk * m->btd.bsz + last * m->btd.bsz + i0 * mb + i0;  // inside B
+        dstride = mb + 1;
+    } else {
+        tan = m->d_band;
+        ntan = m->band_elems;
+        dfirst = nf * (size_t)(m->band_ld + 1) + (size_t)m->half_band;
+        dstride = (size_t)(m->band_ld + 1);
+    }
+    if (dcount == 0) dstride = 1;
+}
+
+// Enqueues Clear (unless `cleared`) + MountLocal/ElementLoads/Loads + MountGlobal
+// and the residual max-norm scan, which leaves the scalar block in h_scal.
+int gf_assemble_enqueue(gf_model *m, bool cleared)
 {
     gf_probe_scope ps(probe_of(m));
     GF_HIP(hipSetDevice(m->device));
     const size_t npad = (size_t)m->npad;
-    double *tan = m->layout == GM_BTD ? (double *)m->btd.A : m->d_band;
-    const size_t ntan = m->layout == GM_BTD ? 3 * (size_t)m->btd.nblk * m->btd.bsz : m->band_elems;
-    // the padding rows [n_free, npad) carry a unit diagonal (all in the last block
-    // row for the block-tridiagonal layout)
-    size_t dfirst, dstride;
-    const size_t dcount = npad - (size_t)m->n_free, nf = (size_t)m->n_free;
-    if (m->layout == GM_BTD) {
-        const size_t mb = (size_t)m->btd.m, last = (size_t)m->btd.nblk - 1, i0 = nf - last * mb;
-        dfirst = (size_t)m->btd.nblk * m->btd.bsz + last * m->btd.bsz + i0 * mb + i0;  // inside B
-        dstride = mb + 1;
-    } else {
-        dfirst = nf * (size_t)(m->band_ld + 1) + (size_t)m->half_band;
-        dstride = (size_t)(m->band_ld + 1);
+    if (!cleared) {
+        double *tan;
+        size_t ntan, dfirst, dstride, dcount;
+        gf_assemble_clear_ranges(m, tan, ntan, dfirst, dstride, dcount);
+        if (m->fronts_on)
+            GF_TRY(gf_launch_clear_csr(m->stream, m->d_r, npad, m->d_scal + GF_SCAL_RES, 8, m->d_band, m->band_ld,
+                                       m->half_band, m->d_csr_ptr, m->d_csr_col, m->n_free));
+        else
+            GF_TRY(gf_launch_clear3(m->stream, m->d_r, npad, tan, ntan, m->d_scal + GF_SCAL_RES, 8, dfirst, dstride,
+                                    dcount));
     }
-    if (m->fronts_on)
-        GF_TRY(gf_launch_clear_csr(m->stream, m->d_r, npad, m->d_scal + GF_SCAL_RES, 8, m->d_band, m->band_ld,
-                                   m->half_band, m->d_csr_ptr, m->d_csr_col, m->n_free));
-    else
-        GF_TRY(gf_launch_clear3(m->stream, m->d_r, npad, tan, ntan, m->d_scal + GF_SCAL_RES, 8, dfirst, dstride, dcount));
     // load time and gravity ramp factor from the scalar block (set by gf_begin_step)
     const double *tp = m->d_scal + GF_SCAL_TIME, *lfp = m->d_scal + GF_SCAL_LF;
     GF_TRY(gf_nodal_loads(m, tp));
@@ -1098,9 +1112,6 @@ int gf_assemble_enqueue(gf_model *m, bool copy_norms)
     m->pending_launches[GF_PH_ASSEMBLE] += nl_beam + nl_shell;
     m->factored = false;
     GF_TRY(gf_scan_residual(m));
-    if (copy_norms)
-        GF_HIP(hipMemcpyAsync(m->h_scal + GF_SCAL_RES, m->d_scal + GF_SCAL_RES, 3 * sizeof(double),
-                              hipMemcpyDeviceToHost, m->stream));
     return GF_OK;
 }
 
@@ -1121,7 +1132,7 @@ int gf_assemble_result(gf_model *m, double *res_out)
 extern "C" int gf_assemble(gf_model *m, double *res_out)
 {
     if (!m) return GF_E_ARG;
-    GF_TRY(gf_assemble_enqueue(m, true));
+    GF_TRY(gf_assemble_enqueue(m, false));
     GF_HIP(hipStreamSynchronize(m->stream));
     double res[3];
     GF_TRY(gf_assemble_result(m, res));
@@ -1129,14 +1140,16 @@ extern "C" int gf_assemble(gf_model *m, double *res_out)
     return GF_OK;
 }
 
-// UpdateDisps, the next iteration's assembly (then_assemble) and one copy of
-// the scalar block, after a solve whose increment is in d_x.
+// UpdateDisps and the next iteration's assembly (then_assemble), after a solve
+// whose increment is in d_x; the scalar block ends up in h_scal.
 static int update_tail_enqueue(gf_model *m, bool then_assemble)
 {
+    if (then_assemble) {
+        GF_TRY(gf_update_clear(m));
+        return gf_assemble_enqueue(m, true);
+    }
     GF_TRY(gf_update_disp(m, false));
-    if (then_assemble) GF_TRY(gf_assemble_enqueue(m, false));
-    const int nscal = then_assemble ? GF_SCAL_RES + 3 : GF_SCAL_FLAG + 1;
-    GF_HIP(hipMemcpyAsync(m->h_scal, m->d_scal, nscal * sizeof(double), hipMemcpyDeviceToHost, m->stream));
+    GF_HIP(hipMemcpyAsync(m->h_scal, m->d_scal, (GF_SCAL_FLAG + 1) * sizeof(double), hipMemcpyDeviceToHost, m->stream));
     return GF_OK;
 }
 
@@ -1302,19 +1315,18 @@ int gf_refine_step(gf_model *m, int *more)
 
 static int solve_fp64_launches(gf_model *m, int &nl_fac, int &nl_sol);
 
-// The whole FP64 Newton iteration -- clear of the increment norms and flag, the
-// factorisation and solve, UpdateDisps, the next iteration's assembly and
-// residual scan, the copy of the scalar block -- captured once per model into a
+// The whole FP64 Newton iteration -- the factorisation and solve, UpdateDisps, the
+// next iteration's assembly and residual scan, the scalar block to the host and
+// the clear of its increment norms and flag -- captured once per model into a
 // graph and replayed on every iteration (the launch sequence depends on the
 // model only; the load time and gravity factor are read from the scalar block).
-// The graph holds kernel and copy nodes, no memset.
+// The graph holds kernel nodes and, with the band LU, a copy; no memset.
 static int iteration_graph_launch(gf_model *m)
 {
     if (!m->iter_graph) {
         GF_HIP(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
         int nf = 0, ns = 0;
-        int st = gf_launch_fill_bytes(m->stream, m->d_scal, (GF_SCAL_FLAG + 1) * sizeof(double));
-        if (!st) st = solve_fp64_launches(m, nf, ns);
+        int st = solve_fp64_launches(m, nf, ns);
         if (!st) st = update_tail_enqueue(m, true);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(m->stream, &g);
@@ -1328,7 +1340,12 @@ static int iteration_graph_launch(gf_model *m)
         if (ei != hipSuccess) m->iter_graph = nullptr;
         GF_HIP(ei);
     }
+    // the norms and flag: left clear by the last iteration's scan unless other work
+    // on the scalar block came between
+    if (!m->scal_clear)
+        GF_TRY(gf_launch_fill_bytes(m->stream, m->d_scal, (GF_SCAL_FLAG + 1) * sizeof(double)));
     GF_HIP(hipGraphLaunch(m->iter_graph, m->stream));
+    m->scal_clear = true;
     m->factored = false;  // the iteration ends with the next assembly
     return GF_OK;
 }
@@ -1355,6 +1372,7 @@ int gf_solve_update_enqueue(gf_model *m, bool then_assemble)
         m->n_direct++;
     }
     if (!mixed && then_assemble && !m->timing && m->use_graph) return iteration_graph_launch(m);
+    m->scal_clear = false;
     GF_TRY(gf_launch_fill_bytes(m->stream, m->d_scal, (GF_SCAL_FLAG + 1) * sizeof(double)));
     if (mixed) {
         m->refine_then_assemble = then_assemble;
@@ -1510,6 +1528,7 @@ extern "C" int gf_solve(gf_model *m, int *info_fail)
     gf_probe_scope ps(probe_of(m));
     GF_HIP(hipSetDevice(m->device));
     *info_fail = 0;
+    m->scal_clear = false;
     GF_TRY(gf_launch_fill_bytes(m->stream, m->d_flag, 4));
     m->n_solves++;
     // Mixed precision backs off after two fallbacks in a row: the next
@@ -1544,6 +1563,7 @@ extern "C" int gf_update(gf_model *m, double *inc_out)
 {
     if (!m) return GF_E_ARG;
     GF_HIP(hipSetDevice(m->device));
+    m->scal_clear = false;
     GF_TRY(gf_update_disp(m, true));
     if (inc_out) {
         GF_HIP(hipMemcpyAsync(m->h_scal, m->d_scal, 5 * sizeof(double), hipMemcpyDeviceToHost, m->stream));

@@ -23,11 +23,11 @@ __global__ void fill_kernel(double *p, size_t n, double v)
 
 // Zeroes three ranges; in the second, the entries dfirst + k dstride (k < dcount)
 // get 1 instead (the unit diagonal of the padding rows of the global matrix).
-__global__ __launch_bounds__(256) void clear3_kernel(double *a, size_t na, double *b, size_t nb, double *c, size_t nc,
-                                                     size_t dfirst, size_t dstride, size_t dcount)
+__device__ __forceinline__ void clear3(size_t gid, size_t step, double *a, size_t na, double *b, size_t nb, double *c,
+                                       size_t nc, size_t dfirst, size_t dstride, size_t dcount)
 {
     const size_t n = na + nb + nc;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+    for (size_t i = gid; i < n; i += step) {
         double *p = i < na ? a + i : i < na + nb ? b + (i - na) : c + (i - na - nb);
         double v = 0.0;
         if (i >= na + dfirst && i < na + nb) {
@@ -37,20 +37,29 @@ __global__ __launch_bounds__(256) void clear3_kernel(double *a, size_t na, doubl
         *p = v;
     }
 }
+__global__ __launch_bounds__(256) void clear3_kernel(double *a, size_t na, double *b, size_t nb, double *c, size_t nc,
+                                                     size_t dfirst, size_t dstride, size_t dcount)
+{
+    clear3(blockIdx.x * (size_t)256 + threadIdx.x, (size_t)gridDim.x * 256, a, na, b, nb, c, nc, dfirst, dstride, dcount);
+}
 
 // Zeroes a and c, and the band entries (row, cols[k]) for k in [ptr[row],
 // ptr[row + 1]) of rows < nrows (the positions the element scatter writes): one
 // wavefront per band row, the short ranges by every thread.
-__global__ __launch_bounds__(256) void clear_csr_kernel(double *a, size_t na, double *c, size_t nc, double *ab,
-                                                         int ld, int hb, const int *ptr, const int *cols, int nrows)
+__device__ __forceinline__ void clear_csr(size_t gid, double *a, size_t na, double *c, size_t nc, double *ab, int ld,
+                                          int hb, const int *ptr, const int *cols, int nrows)
 {
-    const size_t gid = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
     if (gid < na) a[gid] = 0.0;
     if (gid < nc) c[gid] = 0.0;
     const int row = (int)(gid >> 6), lane = threadIdx.x & 63;
     if (row >= nrows) return;
     double *base = ab + (size_t)row * (size_t)ld + (size_t)hb;
     for (int k = ptr[row] + lane; k < ptr[row + 1]; k += 64) base[cols[k]] = 0.0;
+}
+__global__ __launch_bounds__(256) void clear_csr_kernel(double *a, size_t na, double *c, size_t nc, double *ab,
+                                                         int ld, int hb, const int *ptr, const int *cols, int nrows)
+{
+    clear_csr(blockIdx.x * (size_t)256 + threadIdx.x, a, na, c, nc, ab, ld, hb, ptr, cols, nrows);
 }
 
 __global__ void fill_u32_kernel(unsigned *p, size_t n)
@@ -148,9 +157,9 @@ __global__ __launch_bounds__(128) void nodal_loads_kernel(int n_ln, const int *_
 // Max-norms of a vector over band rows split by DOF kind (translation /
 // rotation) plus a non-finite flag.  out (as unsigned long long bits of
 // non-negative doubles): [0] trans, [1] rot, [2] flag.
-__device__ __forceinline__ void amax(unsigned long long *p, double v)
+__device__ __forceinline__ unsigned long long amax(unsigned long long *p, double v)
 {
-    atomicMax(p, (unsigned long long)__double_as_longlong(v));
+    return atomicMax(p, (unsigned long long)__double_as_longlong(v));
 }
 
 // Workgroup max of NV non-negative values (256 lanes): wave shuffles, then LDS
@@ -169,14 +178,24 @@ template <int NV> __device__ __forceinline__ void block_amax(double (&v)[NV], un
     if (threadIdx.x < NV) {
         double mx = sred[0][threadIdx.x];
         for (int w = 1; w < 4; w++) mx = fmax(mx, sred[w][threadIdx.x]);
-        amax(out + threadIdx.x, mx);
+        // the result is waited for: what this wavefront does next comes after the maximum
+        const unsigned long long old = amax(out + threadIdx.x, mx);
+        asm volatile("" ::"v"(old));
     }
 }
 
-// max |r| over translational and rotational free DOFs, and a non-finite flag.
-__global__ __launch_bounds__(256) void scan_kernel(int n, const double *__restrict__ v,
-                                                   const int *__restrict__ row_nc, unsigned long long *out)
+// max |r| over translational and rotational free DOFs, and a non-finite flag, into
+// scal[GF_SCAL_RES ..].  The workgroup that finishes last (a ticket in
+// scal[GF_SCAL_TICKET]; none waits) then writes the scalar block to the host's
+// pinned mirror and clears the increment norms and the failure flag for the next
+// solve: the copy and the fill that did this were two more dependent launches of
+// each Newton iteration (3.9 and 1.6 us).  Only atomics pass between the
+// workgroups, so no fence: one here writes an XCD's whole L2 back (8 us after a
+// 10,000-element assembly).
+__global__ __launch_bounds__(256) void scan_kernel(int n, const double *__restrict__ v, const int *__restrict__ row_nc,
+                                                   unsigned long long *scal, unsigned long long *host)
 {
+    unsigned long long *out = scal + GF_SCAL_RES;
     double m[3] = {0.0, 0.0, 0.0};  // translations, rotations, non-finite
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         double a = fabs(v[i]);
@@ -185,15 +204,26 @@ __global__ __launch_bounds__(256) void scan_kernel(int n, const double *__restri
         else m[1] = fmax(m[1], a);
     }
     block_amax<3>(m, out);
+    // (the wavefront that added this workgroup's maxima takes its ticket)
+    if (threadIdx.x >= 64) return;
+    unsigned ticket = 0;
+    if (threadIdx.x == 0) ticket = atomicAdd((unsigned *)(scal + GF_SCAL_TICKET), 1u);
+    if ((unsigned)__builtin_amdgcn_readfirstlane((int)ticket) != gridDim.x - 1) return;
+    if (threadIdx.x < GF_SCAL_RES + 3) {
+        host[threadIdx.x] = atomicOr(scal + threadIdx.x, 0ull);  // read where the maxima were formed
+        if (threadIdx.x <= GF_SCAL_FLAG) scal[threadIdx.x] = 0;
+    }
+    if (threadIdx.x == 0) scal[GF_SCAL_TICKET] = 0;
 }
 
 // d += x on free DOFs; scans |x| and the updated |d| (CheckGLConvergence).
-__global__ __launch_bounds__(256) void update_kernel(int n, const double *__restrict__ x,
-                                                     const int *__restrict__ row_nc, double *__restrict__ disp,
-                                                     unsigned long long *out)
+// Workgroups `block` of `blocks`.
+__device__ __forceinline__ void update_rows(int block, int blocks, int n, const double *__restrict__ x,
+                                            const int *__restrict__ row_nc, double *__restrict__ disp,
+                                            unsigned long long *out)
 {
     double m[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // |x| t/r, |d| t/r, non-finite
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    for (int i = block * blockDim.x + threadIdx.x; i < n; i += blocks * blockDim.x) {
         int nc = row_nc[i];
         double xi = x[i];
         double dn = disp[nc] + xi;
@@ -204,6 +234,36 @@ __global__ __launch_bounds__(256) void update_kernel(int n, const double *__rest
         else { m[1] = fmax(m[1], ax); m[3] = fmax(m[3], ad); }
     }
     block_amax<5>(m, out);
+}
+__global__ __launch_bounds__(256) void update_kernel(int n, const double *__restrict__ x,
+                                                     const int *__restrict__ row_nc, double *__restrict__ disp,
+                                                     unsigned long long *out)
+{
+    update_rows(blockIdx.x, gridDim.x, n, x, row_nc, disp, out);
+}
+
+// The update and the clear that the next assembly begins with, in one launch
+// (neither touches what the other does): the first `ub` workgroups update, the
+// others clear.  CSR: as clear_csr_kernel, else as clear3_kernel.
+struct ClearArgs {
+    double *a, *b, *c;
+    size_t na, nb, nc;
+    size_t dfirst, dstride, dcount;   // clear3
+    int ld, hb, nrows;                // csr (b: the band)
+    const int *ptr, *cols;
+};
+template <bool CSR>
+__global__ __launch_bounds__(256) void update_clear_kernel(int ub, int n, const double *__restrict__ x,
+                                                           const int *__restrict__ row_nc, double *__restrict__ disp,
+                                                           unsigned long long *out, ClearArgs q)
+{
+    if ((int)blockIdx.x < ub) {
+        update_rows(blockIdx.x, ub, n, x, row_nc, disp, out);
+        return;
+    }
+    const size_t gid = (blockIdx.x - ub) * (size_t)256 + threadIdx.x;
+    if constexpr (CSR) clear_csr(gid, q.a, q.na, q.c, q.nc, q.b, q.ld, q.hb, q.ptr, q.cols, q.nrows);
+    else clear3(gid, (size_t)(gridDim.x - ub) * 256, q.a, q.na, q.b, q.nb, q.c, q.nc, q.dfirst, q.dstride, q.dcount);
 }
 
 // Node::SaveConfiguration: x += u, alpha <- compose(alpha_delta, alpha), Euler vector.
@@ -303,11 +363,13 @@ int gf_nodal_loads(gf_model *m, const double *tp)
     return GF_OK;
 }
 
-// The norms land in d_scal[GF_SCAL_RES..+2], which the assembly's clear zeroed.
+// The norms land in d_scal[GF_SCAL_RES..+2], which the assembly's clear zeroed, and
+// with the rest of the scalar block in h_scal; the increment norms and the flag
+// are zero afterwards.
 int gf_scan_residual(gf_model *m)
 {
     hipLaunchKernelGGL(scan_kernel, dim3(grid_for(m->n_free, 256, 128)), dim3(256), 0, m->stream, m->n_free, m->d_r,
-                       m->d_row_nc, (unsigned long long *)(m->d_scal + GF_SCAL_RES));
+                       m->d_row_nc, (unsigned long long *)m->d_scal, (unsigned long long *)m->h_scal);
     GF_HIP(hipGetLastError());
     return GF_OK;
 }
@@ -321,6 +383,34 @@ int gf_update_disp(gf_model *m, bool zero_norms)
     }
     hipLaunchKernelGGL(update_kernel, dim3(grid_for(m->n_free, 256, 128)), dim3(256), 0, m->stream, m->n_free,
                        m->d_x, m->d_row_nc, m->d_disp, (unsigned long long *)m->d_scal);
+    GF_HIP(hipGetLastError());
+    return GF_OK;
+}
+
+// UpdateDisps (norms cleared by the caller) with the clear of the next assembly.
+int gf_update_clear(gf_model *m)
+{
+    ClearArgs q{};
+    gf_assemble_clear_ranges(m, q.b, q.nb, q.dfirst, q.dstride, q.dcount);
+    q.a = m->d_r;
+    q.na = (size_t)m->npad;
+    q.c = m->d_scal + GF_SCAL_RES;
+    q.nc = 8;
+    const int ub = grid_for(m->n_free, 256, 128);
+    unsigned long long *out = (unsigned long long *)m->d_scal;
+    if (m->fronts_on) {
+        q.ld = m->band_ld;
+        q.hb = m->half_band;
+        q.ptr = m->d_csr_ptr;
+        q.cols = m->d_csr_col;
+        q.nrows = m->n_free;
+        const size_t n = std::max((size_t)q.nrows * 64, std::max(q.na, q.nc));
+        hipLaunchKernelGGL(update_clear_kernel<true>, dim3(ub + (unsigned)((n + 255) / 256)), dim3(256), 0, m->stream, ub,
+                           m->n_free, m->d_x, m->d_row_nc, m->d_disp, out, q);
+    } else {
+        hipLaunchKernelGGL(update_clear_kernel<false>, dim3(ub + grid_for(q.na + q.nb + q.nc, 256)), dim3(256), 0,
+                           m->stream, ub, m->n_free, m->d_x, m->d_row_nc, m->d_disp, out, q);
+    }
     GF_HIP(hipGetLastError());
     return GF_OK;
 }

@@ -208,7 +208,7 @@ int gf_static_run::advance()
 int gf_static_run::enqueue_assemble()
 {
     t_mark = std::chrono::steady_clock::now();
-    int st = gf_assemble_enqueue(m, true);
+    int st = gf_assemble_enqueue(m, false);
     if (st) return st;
     if ((st = record())) return st;
     phase = PH_ASSEMBLED;
