@@ -90,20 +90,48 @@ __global__ __launch_bounds__(ASM_T, 6) void front_assemble_kernel(FrontTab t, in
     constexpr int RS = ASM_T / NB;  // row stride of a thread's rows
     const int cj = c0 + j;
     const int *rows = t.rows + F.rows;
+    // Few tiles (the upper levels, small plates) are a chain of dependent loads:
+    // item, front, child's map, child's entries, and entry list, band.  The two
+    // chains run together: a thread's first PQ list entries are read to the band's
+    // value while the children's maps arrive (a launch of a few tiles 21.5 -> 19.7
+    // us, level 2 of the 64 x 64 plate 29.7 -> 23.6).
+    constexpr int PQ = 2;
+    const int *ol = t.orig + 3 * (size_t)t.asm_orig[2 * (size_t)(first + blockIdx.x)];
+    const int no = t.asm_orig[2 * (size_t)(first + blockIdx.x) + 1];
+    auto entry = [&](int oi, int oc) {
+        const double a = ab[(size_t)oi * (size_t)ld + (size_t)(oc + hb)];
+        return D ? D[oi] * a * D[oc] : a;
+    };
+    int pos[PQ], oi[PQ], oc[PQ];
+#pragma unroll
+    for (int k = 0; k < PQ; k++) {
+        const int q = min(tid + ASM_T * k, max(no - 1, 0));
+        pos[k] = no ? ol[3 * q] : 0;
+        oi[k] = no ? ol[3 * q + 1] : 0;
+        oc[k] = no ? ol[3 * q + 2] : 0;
+    }
     T v[ASM_R];
 #pragma unroll
     for (int r = 0; r < ASM_R; r++) v[r] = T(0);
-    for (int c = F.ch0; c < F.ch1; c++) {
-        const gf_front_dev C = t.fr[t.child[c]];
-        const int *im = t.inv + t.child_inv[c];
-        const int b = im[cj];
+    double pre[PQ];
+    for (int c = F.ch0; c < F.ch1 || c == F.ch0; c++) {
+        const bool have = c < F.ch1;
+        const gf_front_dev C = t.fr[have ? t.child[c] : f];
+        const int *im = t.inv + (have ? t.child_inv[c] : 0);
+        int b = -1, a[ASM_R];
+        if (have) {
+            b = im[cj];
+#pragma unroll
+            for (int r = 0; r < ASM_R; r++) a[r] = im[r0 + i0 + RS * r];
+        }
+        if (c == F.ch0)
+#pragma unroll
+            for (int k = 0; k < PQ; k++) pre[k] = no ? entry(oi[k], oc[k]) : 0.0;
         if (b < 0) continue;
         const T *U = Fb + C.F + (size_t)(NB * C.kb) * C.mp + NB * C.kb + b;
 #pragma unroll
-        for (int r = 0; r < ASM_R; r++) {
-            const int a = im[r0 + i0 + RS * r];
-            if (a >= 0) v[r] += U[(size_t)a * C.mp];
-        }
+        for (int r = 0; r < ASM_R; r++)
+            if (a[r] >= 0) v[r] += U[(size_t)a[r] * C.mp];
     }
     // the children's sums into the tile in LDS, the tile's tangent entries (its
     // precomputed list) added there, then the tile written out row by row
@@ -114,13 +142,12 @@ __global__ __launch_bounds__(ASM_T, 6) void front_assemble_kernel(FrontTab t, in
         sm.P[(i0 + RS * r) * LDT + j] = v[r];
     }
     __syncthreads();
-    const int *ol = t.orig + 3 * (size_t)t.asm_orig[2 * (size_t)(first + blockIdx.x)];
-    const int no = t.asm_orig[2 * (size_t)(first + blockIdx.x) + 1];
-    for (int q = tid; q < no; q += ASM_T) {
-        const int pos = ol[3 * q], oi = ol[3 * q + 1], oc = ol[3 * q + 2];
-        double a = ab[(size_t)oi * (size_t)ld + (size_t)(oc + hb)];
-        if (D) a = D[oi] * a * D[oc];
-        sm.P[(pos >> 6) * LDT + (pos & 63)] += (T)a;
+#pragma unroll
+    for (int k = 0; k < PQ; k++)
+        if (tid + ASM_T * k < no) sm.P[(pos[k] >> 6) * LDT + (pos[k] & 63)] += (T)pre[k];
+    for (int q = tid + ASM_T * PQ; q < no; q += ASM_T) {
+        const int ps = ol[3 * q];
+        sm.P[(ps >> 6) * LDT + (ps & 63)] += (T)entry(ol[3 * q + 1], ol[3 * q + 2]);
     }
     __syncthreads();
     T *out = Fb + F.F + cj;

@@ -291,11 +291,12 @@ template <typename T>
 __device__ __forceinline__ typename mfma<T>::acc_t mm16(const T *P, int lp, const T *Q, int lq)
 {
     const int lane = threadIdx.x & 63;
-    typename mfma<T>::acc_t acc{};
+    typename mfma<T>::acc_t acc[2] = {};  // two chains of two
 #pragma unroll
     for (int k0 = 0; k0 < 16; k0 += 4)
-        acc = mfma<T>::run(P[(lane & 15) * lp + k0 + (lane >> 4)], Q[(k0 + (lane >> 4)) * lq + (lane & 15)], acc);
-    return acc;
+        acc[k0 >> 2 & 1] = mfma<T>::run(P[(lane & 15) * lp + k0 + (lane >> 4)], Q[(k0 + (lane >> 4)) * lq + (lane & 15)],
+                                        acc[k0 >> 2 & 1]);
+    return acc[0] + acc[1];
 }
 
 // Scratch of inverse64: two sets of three saved 16 x 16 column blocks, and one
@@ -334,29 +335,31 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const bool act = tid < 256;
     const PivotGuard<T> pg;
-    // largest magnitude in the block, and the original diagonal
-    if (act) {
-        const int r = tid >> 2, c0 = 16 * (tid & 3);
-        T mx = T(0);
+    auto wave_max = [&](T v) {
 #pragma unroll
-        for (int j = 0; j < 16; j++) mx = fmax(mx, fabs(M[r * LDT + c0 + j]));
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) mx = fmax(mx, __shfl_xor(mx, o));
-        if (lane == 0) aux[wave] = mx;
-        if (tid < NB) aux[4 + tid] = fabs(M[tid * LDT + tid]);
-    }
-    __syncthreads();
-    const T mx = fmax(fmax(aux[0], aux[1]), fmax(aux[2], aux[3]));
-    bool bad = !(mx > T(0)) || !(mx < pg.huge), pert = false;
+        for (int o = 1; o < 64; o <<= 1) v = fmax(v, __shfl_xor(v, o));
+        return v;
+    };
     // wave 0: pivot thresholds of block kb (their reciprocals replace the
     // original diagonal in aux; written and read by this wave only), then the
     // inverse of the block in place
+    bool bad = false, pert = false;
     auto pivot_block = [&](int kb) {
         T *ie = aux + 4 + 16 * kb;
-        if (lane < 16) {
-            const T dk = ie[lane];
-            ie[lane] = rcp_of<T>(pg.rel * (dk > T(0) ? dk : mx));
+        T dk = ie[lane & 15];
+        if (__any(!(dk > T(0)))) {
+            // the largest entry of the original block: while it is still whole, then
+            // from the scan beside the first inverse
+            T mx = T(0);
+            if (kb == 0) {
+                for (int t = lane; t < NB * NB; t += 64) mx = fmax(mx, fabs(M[(t >> 6) * LDT + (t & 63)]));
+                mx = wave_max(mx);
+            } else {
+                for (int k = 0; k < 4; k++) mx = fmax(mx, aux[k]);
+            }
+            dk = dk > T(0) ? dk : mx;
         }
+        if (lane < 16) ie[lane] = rcp_of<T>(pg.rel * dk);
         wave_lds_fence();
         inv16<T>(M + 16 * kb * LDT + 16 * kb, ie, pg.huge, bad, pert);
     };
@@ -378,12 +381,27 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
             if (sv) sv[r * TMP_LD + c] = x;
         }
     };
-    // step 0's pivot block and column blocks
+    // step 0's pivot block and column blocks; beside the pivot block's inverse the
+    // largest magnitudes of the row blocks (wave 0: of its own block), which tell
+    // an all-zero block and one with infinite entries
     if (wave == 0) {
+        aux[4 + lane] = fabs(M[lane * LDT + lane]);
+        T mx = T(0);
+#pragma unroll
+        for (int t = 0; t < 4; t++) mx = fmax(mx, fabs(M[(lane & 15) * LDT + 4 * (lane >> 4) + t]));
+        mx = wave_max(mx);
+        if (lane == 0) aux[0] = mx;
+        wave_lds_fence();
         pivot_block(0);
     } else if (act) {
         const T *src = block(wave, 0);
         for (int t = lane; t < 256; t += 64) tmp[(wave - 1) * CS + (t >> 4) * TMP_LD + (t & 15)] = src[(t >> 4) * LDT + (t & 15)];
+        T mx = T(0);
+        for (int t = lane; t < 16 * NB; t += 64) mx = fmax(mx, fabs(src[(t >> 6) * LDT + (t & 63)]));
+        // row block 0 right of the pivot block
+        for (int t = lane; t < 256; t += 64) mx = fmax(mx, fabs(M[(t >> 4) * LDT + 16 * wave + (t & 15)]));
+        mx = wave_max(mx);
+        if (lane == 0) aux[wave] = mx;
     }
     __syncthreads();
 #pragma unroll 1
@@ -435,6 +453,8 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
         __syncthreads();
     }
     if (tid == 0) {
+        const T mx = fmax(fmax(aux[0], aux[1]), fmax(aux[2], aux[3]));
+        bad |= !(mx > T(0)) || !(mx < pg.huge);
         const int bits = (bad ? 1 : 0) | (pert ? 2 : 0);
         if (bits) atomicOr(flag, bits);
     }
