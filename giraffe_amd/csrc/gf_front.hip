@@ -388,7 +388,7 @@ __global__ __launch_bounds__(256, 3) void front_step_kernel(FrontTab t, int firs
     }
     colchunk_load(l1, Lp, ld, KT);  // behind the second half of product 1
     if (ka > KT) mm_xc<T>(w, sm.X, sm.C, KT, ka);
-    if (kind == 2) {
+    if (__builtin_expect(kind == 2, 1)) {
         acc_each<T>([&](int x, int y, int v, int, int) { at(tile(ti) + acc_at<T>(x, y, v, ld), ao) = w.a[x][y][v]; });
         return;
     }

@@ -511,6 +511,11 @@ struct gf_model {
     int npad = 0;                   // padded system size
     double *d_scal = nullptr;       // small reduction results
     double *h_scal = nullptr;       // pinned mirror
+    // assembly of the shells by rows (gf_shell_gather_setup): elements of each DOF
+    // block, positions of their columns
+    bool shell_gather = false;
+    int *d_sg_ptr = nullptr, *d_sg_list = nullptr;
+    unsigned char *d_sg_pos = nullptr;
     bool scal_clear = false;        // d_scal[0..GF_SCAL_FLAG] is zero once the stream is there
     int *d_flag = nullptr;          // solver failure flag
     bool factored = false;
@@ -566,6 +571,7 @@ int gf_nodal_loads(gf_model *m, const double *tp);
 int gf_scan_residual(gf_model *m);
 int gf_update_disp(gf_model *m, bool zero_norms);
 int gf_update_clear(gf_model *m);
+int gf_shell_gather_setup(gf_model *m, const std::vector<int> &conn);
 // The tangent's storage and, as clear3 takes it, the unit diagonal of its padding rows.
 void gf_assemble_clear_ranges(const gf_model *m, double *&tan, size_t &ntan, size_t &dfirst, size_t &dstride,
                               size_t &dcount);

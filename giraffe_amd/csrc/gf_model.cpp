@@ -170,7 +170,7 @@ static void release(gf_model *m)
                     m->d_scal, m->d_copy0, m->d_bgp0, m->d_sconn, m->d_sconst, m->d_spconst, m->d_sgp,
                     m->d_sgp0, m->d_spload, m->d_spflag, m->d_band, m->d_swork, m->d_band_inv, m->d_bbuoy,
                     m->d_front, m->d_front_e, m->d_front_v, m->d_csr_ptr, m->d_csr_col, m->d_shell_rec,
-                    m->d_shell_prec, m->d_shell_K, m->d_shell_f};
+                    m->d_shell_prec, m->d_shell_K, m->d_shell_f, m->d_sg_ptr, m->d_sg_list, m->d_sg_pos};
     for (void *b : bufs) gf_pool_free(b);
     gf_front_free(m->fronts);
     if (m->h_scal) gf_pinned_free(m->h_scal);
@@ -496,6 +496,7 @@ static size_t footprint(const gf_model_desc *d, const gf_model *m, int precision
     b += nb * (3 * 4 + BC_COUNT * 8 + 2 * BG_COUNT * 8 + 8);                  // Beam_1 / Pipe_1 records
     b += ns * (6 * 4 + SC_COUNT * 8 + SP_COUNT * 8 + 2 * SG_COUNT * 8 + 8);   // Shell_1 records
     b += ns * (3 * 276 + 6 * 57 + 729 + 27) * 8;                               // Shell_1 assembly records
+    if (m->fronts_on && nb == 0) b += ns * (9 * 4 + 243) + 2 * nn * 4;         // and its tables by rows
     size_t items = d->n_loads ? (size_t)d->load_set_off[d->n_loads] : 0;
     size_t rows = d->n_loads ? (size_t)d->load_tab_off[d->n_loads] : 0;
     b += (size_t)d->n_loads * NL_REC * 8 + items * 12 + rows * 7 * 8;         // loads and tables
@@ -636,9 +637,10 @@ static int create(const gf_model_desc *d, const gf_options *opt, gf_model *m)
         }
     }
     // shells, colour-sorted SoA
+    std::vector<int> sconn;  // shell connectivity in colour order
     if (ns > 0) {
         size_t ld = (size_t)ns;
-        std::vector<int> conn(6 * ld);
+        sconn.resize(6 * ld);
         std::vector<double> cst(SC_COUNT * ld), pcs(SP_COUNT * ld), gps(SG_COUNT * ld);
         std::vector<double> rec(SC_COUNT), prec(SP_COUNT), g0(SG_COUNT);
         for (int s2 = 0; s2 < ns; s2++) {
@@ -650,14 +652,14 @@ static int create(const gf_model_desc *d, const gf_options *opt, gf_model *m)
             for (int k = 0; k < SC_COUNT; k++) cst[k * ld + s2] = rec[k];
             for (int k = 0; k < SP_COUNT; k++) pcs[k * ld + s2] = prec[k];
             for (int k = 0; k < SG_COUNT; k++) gps[k * ld + s2] = g0[k];
-            for (int a = 0; a < 6; a++) conn[a * ld + s2] = d->shell_conn[6 * e + a];
+            for (int a = 0; a < 6; a++) sconn[a * ld + s2] = d->shell_conn[6 * e + a];
         }
-        GF_TRY(dalloc(&m->d_sconn, conn.size()));
+        GF_TRY(dalloc(&m->d_sconn, sconn.size()));
         GF_TRY(dalloc(&m->d_sconst, cst.size()));
         GF_TRY(dalloc(&m->d_spconst, pcs.size()));
         GF_TRY(dalloc(&m->d_sgp, gps.size()));
         GF_TRY(dalloc(&m->d_sgp0, gps.size()));
-        GF_TRY(upload(m, m->d_sconn, conn.data(), conn.size()));
+        GF_TRY(upload(m, m->d_sconn, sconn.data(), sconn.size()));
         GF_TRY(upload(m, m->d_sconst, cst.data(), cst.size()));
         GF_TRY(upload(m, m->d_spconst, pcs.data(), pcs.size()));
         GF_TRY(upload(m, m->d_sgp, gps.data(), gps.size()));
@@ -776,6 +778,7 @@ static int create(const gf_model_desc *d, const gf_options *opt, gf_model *m)
         const size_t nfr = (size_t)m->n_free;
         GF_TRY(gf_launch_clear3(m->stream, nullptr, 0, m->d_band, m->band_elems, nullptr, 0,
                                 nfr * (size_t)(m->band_ld + 1) + (size_t)hb, (size_t)(m->band_ld + 1), npad - nfr));
+        GF_TRY(gf_shell_gather_setup(m, sconn));
     } else {
         m->band_ld = hb + gf_band_ku(hb);
         m->band_elems = npad * (size_t)(m->band_ld + 1);
@@ -1084,14 +1087,14 @@ void gf_assemble_clear_ranges(const gf_model *m, double *&tan, size_t &ntan, siz
     if (dcount == 0) dstride = 1;
 }
 
-// Enqueues Clear (unless `cleared`) + MountLocal/ElementLoads/Loads + MountGlobal
+// Enqueues Clear (unless `cleared`, or the assembly needs none) + MountLocal/ElementLoads/Loads + MountGlobal
 // and the residual max-norm scan, which leaves the scalar block in h_scal.
 int gf_assemble_enqueue(gf_model *m, bool cleared)
 {
     gf_probe_scope ps(probe_of(m));
     GF_HIP(hipSetDevice(m->device));
     const size_t npad = (size_t)m->npad;
-    if (!cleared) {
+    if (!cleared && !m->shell_gather) {
         double *tan;
         size_t ntan, dfirst, dstride, dcount;
         gf_assemble_clear_ranges(m, tan, ntan, dfirst, dstride, dcount);
@@ -1104,11 +1107,13 @@ int gf_assemble_enqueue(gf_model *m, bool cleared)
     }
     // load time and gravity ramp factor from the scalar block (set by gf_begin_step)
     const double *tp = m->d_scal + GF_SCAL_TIME, *lfp = m->d_scal + GF_SCAL_LF;
-    GF_TRY(gf_nodal_loads(m, tp));
+    // (the assembly by rows writes where the others add, so it comes first)
+    if (!m->shell_gather) GF_TRY(gf_nodal_loads(m, tp));
     tick(m, GF_PH_ASSEMBLE, true);
     GF_TRYN(nl_beam, gf_beam_assemble(m, lfp));
     GF_TRYN(nl_shell, gf_shell_assemble(m, lfp, tp));
     tick(m, GF_PH_ASSEMBLE, false);
+    if (m->shell_gather) GF_TRY(gf_nodal_loads(m, tp));
     m->pending_launches[GF_PH_ASSEMBLE] += nl_beam + nl_shell;
     m->factored = false;
     GF_TRY(gf_scan_residual(m));

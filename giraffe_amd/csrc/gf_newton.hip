@@ -390,6 +390,7 @@ int gf_update_disp(gf_model *m, bool zero_norms)
 // UpdateDisps (norms cleared by the caller) with the clear of the next assembly.
 int gf_update_clear(gf_model *m)
 {
+    if (m->shell_gather) return gf_update_disp(m, false);  // (needs no clear)
     ClearArgs q{};
     gf_assemble_clear_ranges(m, q.b, q.nb, q.dfirst, q.dstride, q.dcount);
     q.a = m->d_r;

@@ -19,8 +19,10 @@
 // runs for all elements in one launch with every lane busy (shell_record_kernel),
 // the follower pressure's terms likewise (shell_pressure_record_kernel), then one
 // launch of phases 2-4 for all elements writes each element's K and f to HBM,
-// and a light scatter launch per colour (shell_scatter_kernel) adds them, with the
-// pressure terms and the self-weight, into the tangent and residual.
+// and they are added, with the pressure terms and the self-weight, into the tangent
+// and residual: gathered by rows where the tangent's structure is at hand
+// (shell_gather_kernel), else by a light scatter launch per colour
+// (shell_scatter_kernel).
 //   phase 1  lane per (element, gp): kinematics, 3-point thickness integration
 //   phase 2  lane per (element, gp, block RS): the 25 blocks of M
 //   phase 3  lane per (element, I, J): K_IJ, rotated to global
@@ -440,8 +442,8 @@ __global__ __launch_bounds__(SWG, PRE ? 3 : 1) void shell_element_kernel(
 // Follower pressure (MountShellSpecialLoads), lane per (element, u-node a) over all
 // elements: the record out[(6 e + a) SPR ...] holds the unbalanced-force change P_a
 // (3) and the load stiffness rows of node a (3 x 18, global frame); zeros for an
-// element without pressure.  The colour launches of shell_scatter_kernel add them
-// to the element's own scatter.
+// element without pressure.  The assembly (by rows or by colour) adds them to
+// the element's own.
 __global__ __launch_bounds__(256) void shell_pressure_record_kernel(
     int ns, size_t ld, const int *__restrict__ conn, const double *__restrict__ cst,
     const double *__restrict__ pc, const double *__restrict__ disp, const double *__restrict__ copy,
@@ -795,6 +797,173 @@ __global__ __launch_bounds__(256) void shell_scatter_kernel(int e0, int e1, size
     vec_add_n<3>(r, R3, V3);
 }
 
+// ---- assembly by rows -------------------------------------------------------------
+// Where the tangent's structure is at hand (multifrontal models of shells alone),
+// the element matrices are gathered instead of scattered: one wavefront a DOF
+// block (three rows: a node's displacements, or a mid-side node's rotations) adds
+// its elements' rows in LDS, in the colour order of the scatter, and writes its
+// three rows of the band and of the residual once.  One launch, no read of the
+// band and no clear before it, in place of a clear and a scatter launch per
+// colour that each read and write what they add to: 64 x 64 plate 30 + 75 us ->
+// 60 us (bound by the band's writes, 24 or 48 bytes apart from the next), 13 x 13
+// plate 5 + 36 -> 8 us (the chain list, matrix, LDS of one wavefront).  Beams share
+// their DOFs with shells in no order of their own, and the block-tridiagonal form
+// has no list of columns: both keep the scatter.
+
+constexpr int SGMAX = 255;  // columns of a row (positions are bytes; 255: constrained)
+
+// Position of every element matrix column in its row's list of columns, once per
+// model: pos[(9 e + I) 27 + l] for column l of the rows of DOF block I.
+__global__ __launch_bounds__(256) void shell_pos_kernel(int ns, size_t ld, const int *__restrict__ conn,
+                                                        const int *__restrict__ dof, const int *__restrict__ ptr,
+                                                        const int *__restrict__ cols, unsigned char *__restrict__ pos)
+{
+    const size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    if (t >= 243 * (size_t)ns) return;
+    const int e = (int)(t / 243), I = (int)(t - 243 * (size_t)e) / 27, l = (int)(t % 27);
+    int n, c0, nj, cj;
+    dof_block(conn, ld, e, I, n, c0);
+    dof_block(conn, ld, e, l / 3, nj, cj);
+    int row = -1;
+    for (int i = 2; i >= 0; i--) row = dof[6 * n + c0 + i] >= 0 ? dof[6 * n + c0 + i] : row;
+    const int c = dof[6 * nj + cj + l % 3];
+    int p = 255;
+    if (row >= 0 && c >= 0) {
+        int lo = ptr[row], hi = ptr[row + 1];
+        const int first = lo;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (cols[mid] < c) lo = mid + 1;
+            else hi = mid;
+        }
+        p = lo - first;
+    }
+    pos[t] = (unsigned char)p;
+}
+
+// list[ptr[b] .. ptr[b + 1]): the (16 e + I) of DOF block b = 2 node + (rotations),
+// e ascending; the elements are sorted by colour.  res: the residual norms to clear.
+// Loads of SGU elements are in flight at once: a wavefront has no other work beside
+// the six or so elements of its node (one at a time: 65 us at 64 x 64, 10.5 at 13 x 13).
+constexpr int SGU = 4;
+
+template <bool PRESS>
+__global__ __launch_bounds__(256) void shell_gather_kernel(
+    int nblk, size_t ld, const int *__restrict__ bptr, const int *__restrict__ list,
+    const unsigned char *__restrict__ pos, const double *__restrict__ cst, const int *__restrict__ dof,
+    const int *__restrict__ ptr, const int *__restrict__ cols, double *__restrict__ ab, int bld, int hb,
+    double *__restrict__ r, const double *__restrict__ Ke, const double *__restrict__ fe,
+    const double *__restrict__ ppre, const double *__restrict__ lfp, double gx, double gy, double gz, double *res)
+{
+    __shared__ double sm[4][3 * SGMAX];
+    if (blockIdx.x == 0 && threadIdx.x < 8) res[threadIdx.x] = 0.0;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x * 4 + wave;
+    if (b >= nblk) return;  // (no barrier below: a wavefront works by itself)
+    const int q0 = bptr[b], n = bptr[b + 1] - q0;
+    if (n == 0) return;  // (no free DOF either: an element activates what it adds to)
+    int R[3], row = -1;
+#pragma unroll
+    for (int i = 2; i >= 0; i--) {
+        R[i] = dof[3 * b + i];
+        row = R[i] >= 0 ? R[i] : row;
+    }
+    if (row < 0) return;
+    double *acc = sm[wave];
+    const int p0 = ptr[row], len = ptr[row + 1] - p0;
+    const double lf = lfp ? *lfp : 0.0;
+    for (int t = lane; t < 3 * len; t += 64) acc[t] = 0.0;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // the 81 entries of an element's three rows: lane t takes t and t + 64
+    const int i0 = lane / 27, l0 = lane - 27 * i0, l1 = lane + 10;  // (t + 64 = 2 * 27 + (t + 10))
+    const bool two = lane < 17, vec = lane < 3;
+    const double gl = (lane == 0 ? gx : 0.0) + (lane == 1 ? gy : 0.0) + (lane == 2 ? gz : 0.0);
+    double rv = 0.0;
+    for (int q = 0; q < n; q += SGU) {
+        int el[SGU], c0[SGU], c1[SGU];
+        double k0[SGU], k1[SGU], f[SGU], a0[SGU], a1[SGU], af[SGU];
+#pragma unroll
+        for (int u = 0; u < SGU; u++) el[u] = list[q0 + min(q + u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < SGU; u++) {
+            const int e = el[u] >> 4, I = el[u] & 15;
+            const double *K = Ke + (size_t)e * 729 + 81 * I;
+            const unsigned char *ps = pos + (size_t)(9 * (size_t)e + I) * 27;
+            k0[u] = K[lane];
+            k1[u] = K[two ? lane + 64 : lane];
+            f[u] = fe[(size_t)e * 27 + 3 * I + (vec ? lane : 0)];
+            c0[u] = ps[l0];
+            c1[u] = ps[two ? l1 : l0];
+            if (PRESS) {
+                // (rotations carry no pressure: their slots read block 5's and drop it)
+                const double *kp = ppre + ((size_t)e * 6 + min(I, 5)) * SPR;
+                a0[u] = kp[l0 < 18 ? 3 + 18 * i0 + l0 : 0];
+                a1[u] = kp[two && l1 < 18 ? 3 + 36 + l1 : 0];
+                af[u] = kp[vec ? lane : 0];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < SGU; u++) {
+            if (q + u >= n) break;
+            const int e = el[u] >> 4, I = el[u] & 15;
+            if (PRESS && I < 6) {
+                if (l0 < 18) k0[u] += a0[u];
+                if (l1 < 18) k1[u] += a1[u];
+            }
+            if (I < 6 && lf != 0.0) {
+                // self-weight, accumulated twice as src/Shell_1.cpp:1340-1375 does
+                const double mult = lf * cst[SC_RHO * ld + e] * cst[SC_THICK * ld + e];
+                const double gw = cst[(SC_GW + I) * ld + e];
+                for (int rep = 0; rep < 2; rep++) f[u] -= gw * mult * gl;
+            }
+            // (different lanes hold different entries of the three rows)
+            if (c0[u] != 255) acc[i0 * len + c0[u]] += k0[u];
+            if (two && c1[u] != 255) acc[2 * len + c1[u]] += k1[u];
+            rv -= f[u];
+            if (PRESS && I < 6) rv -= af[u];
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        if (R[i] < 0) continue;
+        double *base = ab + (size_t)R[i] * (size_t)bld + (size_t)hb;
+        for (int k = lane; k < len; k += 64) base[cols[p0 + k]] = acc[i * len + k];
+        if (lane == i) r[R[i]] = rv;
+    }
+}
+
+// The tables of the assembly by rows; conn as uploaded (colour order).
+int gf_shell_gather_setup(gf_model *m, const std::vector<int> &conn)
+{
+    const size_t ns = (size_t)m->ns, nb2 = 2 * (size_t)m->nn;
+    int longest = 0;
+    for (size_t i = 0; i + 1 < m->csr_ptr.size(); i++) longest = std::max(longest, m->csr_ptr[i + 1] - m->csr_ptr[i]);
+    if (!m->fronts_on || m->nb > 0 || m->ns == 0 || longest > SGMAX) return GF_OK;
+    std::vector<int> ptr(nb2 + 1, 0), list(9 * ns);
+    auto block = [&](size_t e, int I) { return 2 * (size_t)conn[(I < 6 ? I : I - 3) * ns + e] + (I < 6 ? 0 : 1); };
+    for (size_t e = 0; e < ns; e++)
+        for (int I = 0; I < 9; I++) ptr[block(e, I) + 1]++;
+    for (size_t b = 0; b < nb2; b++) ptr[b + 1] += ptr[b];
+    std::vector<int> at(ptr.begin(), ptr.end() - 1);
+    for (size_t e = 0; e < ns; e++)
+        for (int I = 0; I < 9; I++) list[at[block(e, I)]++] = (int)(16 * e) + I;
+    GF_TRY(gf_pool_alloc((void **)&m->d_sg_ptr, ptr.size() * 4));
+    GF_TRY(gf_pool_alloc((void **)&m->d_sg_list, list.size() * 4));
+    GF_TRY(gf_pool_alloc((void **)&m->d_sg_pos, 243 * ns));
+    GF_HIP(hipMemcpyAsync(m->d_sg_ptr, ptr.data(), ptr.size() * 4, hipMemcpyHostToDevice, m->stream));
+    GF_HIP(hipMemcpyAsync(m->d_sg_list, list.data(), list.size() * 4, hipMemcpyHostToDevice, m->stream));
+    hipLaunchKernelGGL(shell_pos_kernel, dim3((unsigned)((243 * ns + 255) / 256)), dim3(256), 0, m->stream, m->ns, ns,
+                       m->d_sconn, m->d_dof, m->d_csr_ptr, m->d_csr_col, m->d_sg_pos);
+    GF_HIP(hipGetLastError());
+    // the rows that no DOF has stay as they are from here on
+    GF_TRY(gf_launch_fill(m->stream, m->d_r, (size_t)m->npad, 0.0));
+    GF_HIP(hipStreamSynchronize(m->stream));  // (the uploads' host arrays end here)
+    m->shell_gather = true;
+    return GF_OK;
+}
+
 // ---- launchers --------------------------------------------------------------
 int gf_shell_assemble(gf_model *m, const double *lfp, const double *tp)
 {
@@ -802,7 +971,7 @@ int gf_shell_assemble(gf_model *m, const double *lfp, const double *tp)
     int ncol = (int)m->shell_color_off.size() - 1;
     int launches = 0;
     if (m->ns == 0) return 0;
-    // phase 1 of every element and the pressure terms, then one scatter launch per colour
+    // phase 1 of every element and the pressure terms
     hipLaunchKernelGGL(shell_record_kernel, dim3((3 * m->ns + REC_LANES - 1) / REC_LANES), dim3(REC_LANES), 0,
                        m->stream, m->ns, ld, m->d_sconn, m->d_sconst, m->d_sgp, m->d_disp, m->d_shell_rec);
     launches++;
@@ -812,7 +981,8 @@ int gf_shell_assemble(gf_model *m, const double *lfp, const double *tp)
                            m->d_spload, m->d_spflag, m->d_lrec, m->d_tab_t, m->d_tab_v, tp, m->d_shell_prec);
         launches++;
     }
-    // every element's K and f (phases 2-4 from the records), then one scatter launch per colour
+    // every element's K and f (phases 2-4 from the records), then their sum by rows or one
+    // scatter launch per colour
     {
         const int pr = gf_probe_begin(m->stream, GF_KC_SHELL_ASSEMBLE);
         hipLaunchKernelGGL(shell_element_kernel<true>, dim3((m->ns + SEPB - 1) / SEPB), dim3(SWG), 0, m->stream, 0,
@@ -822,6 +992,16 @@ int gf_shell_assemble(gf_model *m, const double *lfp, const double *tp)
         launches++;
     }
     const double *ppre = m->any_pressure ? m->d_shell_prec : nullptr;
+    if (m->shell_gather) {
+        hipLaunchKernelGGL(ppre ? shell_gather_kernel<true> : shell_gather_kernel<false>, dim3((2 * m->nn + 3) / 4),
+                           dim3(256), 0, m->stream, 2 * m->nn, ld, (const int *)m->d_sg_ptr,
+                           (const int *)m->d_sg_list, (const unsigned char *)m->d_sg_pos, m->d_sconst, m->d_dof,
+                           (const int *)m->d_csr_ptr, (const int *)m->d_csr_col, m->d_band, m->band_ld, m->half_band,
+                           m->d_r, (const double *)m->d_shell_K, (const double *)m->d_shell_f, ppre, lfp,
+                           m->gravity[0], m->gravity[1], m->gravity[2], m->d_scal + GF_SCAL_RES);
+        GF_HIP(hipGetLastError());
+        return launches + 1;
+    }
     for (int c = 0; c < ncol; c++) {
         int e0 = m->shell_color_off[c], e1 = m->shell_color_off[c + 1];
         if (e1 <= e0) continue;

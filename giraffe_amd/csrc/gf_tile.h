@@ -352,6 +352,7 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
             // from the scan beside the first inverse
             T mx = T(0);
             if (kb == 0) {
+#pragma unroll 1
                 for (int t = lane; t < NB * NB; t += 64) mx = fmax(mx, fabs(M[(t >> 6) * LDT + (t & 63)]));
                 mx = wave_max(mx);
             } else {
@@ -395,10 +396,13 @@ template <typename T> __device__ __forceinline__ void inverse64(T *M, T *tmp, T 
         pivot_block(0);
     } else if (act) {
         const T *src = block(wave, 0);
+#pragma unroll 2
         for (int t = lane; t < 256; t += 64) tmp[(wave - 1) * CS + (t >> 4) * TMP_LD + (t & 15)] = src[(t >> 4) * LDT + (t & 15)];
         T mx = T(0);
+#pragma unroll 2
         for (int t = lane; t < 16 * NB; t += 64) mx = fmax(mx, fabs(src[(t >> 6) * LDT + (t & 63)]));
         // row block 0 right of the pivot block
+#pragma unroll 2
         for (int t = lane; t < 256; t += 64) mx = fmax(mx, fabs(M[(t >> 4) * LDT + 16 * wave + (t & 15)]));
         mx = wave_max(mx);
         if (lane == 0) aux[wave] = mx;
