@@ -15,7 +15,8 @@
 // block row: (R, R) and (R, 4)).
 //
 // Workgroup: 256 lanes, SEPB = 4 elements; LDS holds per Gauss point the
-// 16 blocks of D, Psi, G, M and Psi^T sigma (48 KB).  In the Newton loop phase 1
+// 16 blocks of D, Psi, G, M and Psi^T sigma (48 KB), and the elements' constants.
+// In the Newton loop phase 1
 // runs for all elements in one launch with every lane busy (shell_record_kernel),
 // the follower pressure's terms likewise (shell_pressure_record_kernel), then one
 // launch of phases 2-4 for all elements writes each element's K and f to HBM,
@@ -25,7 +26,7 @@
 // (shell_scatter_kernel).
 //   phase 1  lane per (element, gp): kinematics, 3-point thickness integration
 //   phase 2  lane per (element, gp, block RS): the 25 blocks of M
-//   phase 3  lane per (element, I, J): K_IJ, rotated to global
+//   phase 3  lane per (element, I, J), a wavefront's of one form: K_IJ, rotated to global
 //   phase 4  lane per (element, I): internal force
 #include "gf_internal.h"
 #include "gf_device.h"
@@ -192,22 +193,6 @@ __device__ __forceinline__ ShellPt shell_point(const ShellKin &k, double mu, dou
     return p;
 }
 
-// Column block I of dN: rows (R) and their coefficients at Gauss point gp.
-__device__ __forceinline__ int col_rows(const double *__restrict__ cst, size_t ld, int e, int gp, int I, int *R,
-                                         double *c)
-{
-    if (I < 6) {
-        R[0] = 0; c[0] = cst[(SC_NU1 + 6 * gp + I) * ld + e];
-        R[1] = 2; c[1] = cst[(SC_NU2 + 6 * gp + I) * ld + e];
-        return 2;
-    }
-    int b = I - 6;
-    R[0] = 1; c[0] = cst[(SC_NA1 + 3 * gp + b) * ld + e];
-    R[1] = 3; c[1] = cst[(SC_NA2 + 3 * gp + b) * ld + e];
-    R[2] = 4; c[2] = cst[(SC_NA + 3 * gp + b) * ld + e];
-    return 3;
-}
-
 // DOF block I of an element -> (node, first component)
 __device__ __forceinline__ void dof_block(const int *__restrict__ conn, size_t ld, int e, int I, int &node, int &c0)
 {
@@ -215,76 +200,97 @@ __device__ __forceinline__ void dof_block(const int *__restrict__ conn, size_t l
     else { node = conn[(3 + I - 6) * ld + e]; c0 = 3; }
 }
 
-// Phase 1 of Shell_1::Mount for one (element, Gauss point): kinematics, the
-// 3-point thickness integration, and the record o[0 .. L_M) (D, Psi, G blocks
-// and Psi^T sigma) that the later phases read.  The D blocks, accumulated over
-// the thickness points, go to oD[0 .. 144) (o + L_D, or scratch of their own
-// that the caller copies into the record); the rest is written once, into o.
-__device__ __forceinline__ void shell_gp_record(const double *__restrict__ cst, const double *__restrict__ gps,
-                                                size_t ld, int e, int gp, const double *__restrict__ disp,
-                                                const int *__restrict__ conn, double *oD, double *o)
+// Phase 1 of Shell_1::Mount for one (element, Gauss point) in two parts: the
+// 3-point thickness integration, which writes the D blocks oD[0 .. 144) and the
+// stress resultants, and the rest of the record (Psi, G blocks, Psi^T sigma) that
+// the later phases read, o[L_P .. L_M).
+//
+// The D blocks are sums over the points of w zeta^p C (p = 0, 1, 2) with C11, C12,
+// C22 full only in their upper 2 x 2 and (2, 2): 32 sums in registers and one write
+// of each entry, instead of 3 x 144 read-modify-writes of LDS.
+struct ShellRes {
+    v3<double> n1, n2, m1, m2;
+};
+__device__ __forceinline__ void shell_gp_moduli(const double *__restrict__ cst, size_t ld, int e, const ShellKin &k,
+                                                double *oD, ShellRes &sr)
 {
-    ShellKin k;
-    shell_kin(cst, gps, ld, e, gp, disp, conn, k);
     const double mu = cst[SC_MU * ld + e], la = cst[SC_LAMBDA * ld + e], th = cst[SC_THICK * ld + e];
     const double drill = cst[SC_DRILL * ld + e];
-    for (int i = 0; i < 144; i++) oD[i] = 0.0;
     v3<double> n1 = mk3(0.0, 0.0, 0.0), n2 = n1, m1 = n1, m2 = n1;
     const double xi[3] = {-0.77459666924148337703585307995648, 0.0, 0.77459666924148337703585307995648};
     const double wt[3] = {0.55555555555555555555555555555556, 0.88888888888888888888888888888889,
                           0.55555555555555555555555555555556};
     const double J = th / 2.0;
+    m3<double> C11[3], C12[3], C22[3];
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+#pragma unroll
+        for (int i = 0; i < 9; i++) C11[p].a[i] = C12[p].a[i] = C22[p].a[i] = 0.0;
+#pragma unroll
     for (int q = 0; q < 3; q++) {
         double zeta = th * xi[q] / 2.0;
         const ShellPt pt = shell_point(k, mu, la, zeta);
         const double g11 = pt.g11, g12 = pt.g12, g21 = pt.g21, g22 = pt.g22, v = pt.v, dv = pt.dv;
         const v3<double> tau1 = pt.tau1, tau2 = pt.tau2;
-        m3<double> C11, C22, C12, C21;
-#pragma unroll
-        for (int i = 0; i < 9; i++) C11.a[i] = C22.a[i] = C12.a[i] = 0.0;
-        C11.a[0] = mu * ((1.0 + g22) * (1.0 + g22) * dv + 1.0);
-        C11.a[1] = -mu * (1.0 + g22) * g21 * dv;
-        C11.a[3] = -mu * (1.0 + g22) * g21 * dv;
-        C11.a[4] = mu * (g21 * g21 * dv + 1.0);
-        C11.a[8] = mu;
-        C22.a[0] = mu * (g12 * g12 * dv + 1.0);
-        C22.a[1] = -mu * ((1.0 + g11) * g12 * dv);
-        C22.a[3] = -mu * ((1.0 + g11) * g12 * dv);
-        C22.a[4] = mu * ((1.0 + g11) * (1.0 + g11) * dv + 1.0);
-        C22.a[8] = mu;
-        C12.a[0] = -mu * ((1.0 + g22) * g12 * dv);
-        C12.a[1] = mu * (v - 1.0 + (1.0 + g11) * (1.0 + g22) * dv);
-        C12.a[3] = mu * (1.0 - v + g12 * g21 * dv);
-        C12.a[4] = -mu * ((1.0 + g11) * g21 * dv);
-        C21 = tr3(C12);
+        const double a0 = mu * ((1.0 + g22) * (1.0 + g22) * dv + 1.0), a1 = -mu * (1.0 + g22) * g21 * dv,
+                     a4 = mu * (g21 * g21 * dv + 1.0);
+        const double c0 = mu * (g12 * g12 * dv + 1.0), c1 = -mu * ((1.0 + g11) * g12 * dv),
+                     c4 = mu * ((1.0 + g11) * (1.0 + g11) * dv + 1.0);
+        const double b0 = -mu * ((1.0 + g22) * g12 * dv), b1 = mu * (v - 1.0 + (1.0 + g11) * (1.0 + g22) * dv),
+                     b3 = mu * (1.0 - v + g12 * g21 * dv), b4 = -mu * ((1.0 + g11) * g21 * dv);
         double w = wt[q] * J;
-        acc3(oD + 9 * 0, w, C11);            // dn1/deta1
-        acc3(oD + 9 * 1, -w * zeta, mE3(C11)); // dn1/dk1
-        acc3(oD + 9 * 2, w, C12);            // dn1/deta2
-        acc3(oD + 9 * 3, -w * zeta, mE3(C12)); // dn1/dk2
-        acc3(oD + 9 * 4, w * zeta, E3m(C11));  // dm1/deta1
-        acc3(oD + 9 * 5, -w * zeta * zeta, mE3(E3m(C11)));
-        acc3(oD + 9 * 6, w * zeta, E3m(C12));
-        acc3(oD + 9 * 7, -w * zeta * zeta, mE3(E3m(C12)));
-        acc3(oD + 9 * 8, w, C21);            // dn2/deta1
-        acc3(oD + 9 * 9, -w * zeta, mE3(C21));
-        acc3(oD + 9 * 10, w, C22);
-        acc3(oD + 9 * 11, -w * zeta, mE3(C22));
-        acc3(oD + 9 * 12, w * zeta, E3m(C21)); // dm2/deta1
-        acc3(oD + 9 * 13, -w * zeta * zeta, mE3(E3m(C21)));
-        acc3(oD + 9 * 14, w * zeta, E3m(C22));
-        acc3(oD + 9 * 15, -w * zeta * zeta, mE3(E3m(C22)));
+        const double wz[3] = {w, w * zeta, w * zeta * zeta};
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            C11[p].a[0] += wz[p] * a0;
+            C11[p].a[1] += wz[p] * a1;
+            C11[p].a[4] += wz[p] * a4;
+            C12[p].a[0] += wz[p] * b0;
+            C12[p].a[1] += wz[p] * b1;
+            C12[p].a[3] += wz[p] * b3;
+            C12[p].a[4] += wz[p] * b4;
+            C22[p].a[0] += wz[p] * c0;
+            C22[p].a[1] += wz[p] * c1;
+            C22[p].a[4] += wz[p] * c4;
+        }
+        C11[0].a[8] += w * mu;  // (E3's products drop it where zeta stands)
         n1 = add3(n1, scl3(w, tau1));
         n2 = add3(n2, scl3(w, tau2));
         // e3 x tau = (-tau.y, tau.x, 0)
         m1 = add3(m1, scl3(w * zeta, mk3(-tau1.y, tau1.x, 0.0)));
         m2 = add3(m2, scl3(w * zeta, mk3(-tau2.y, tau2.x, 0.0)));
     }
+    C22[0].a[8] = C11[0].a[8];
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        C11[p].a[3] = C11[p].a[1];
+        C22[p].a[3] = C22[p].a[1];
+    }
+    auto blocks = [](double *o, const m3<double> &X0, const m3<double> &X1, const m3<double> &X2)
+        __attribute__((always_inline)) {
+        st3(o + 9 * 0, X0);                              // dn/deta
+        st3(o + 9 * 1, mscl(-1.0, mE3(X1)));             // dn/dk
+        st3(o + 9 * 4, E3m(X1));                         // dm/deta
+        st3(o + 9 * 5, mscl(-1.0, mE3(E3m(X2))));        // dm/dk
+    };
+    blocks(oD + 9 * 0, C11[0], C11[1], C11[2]);
+    blocks(oD + 9 * 2, C12[0], C12[1], C12[2]);
+    blocks(oD + 9 * 8, tr3(C12[0]), tr3(C12[1]), tr3(C12[2]));
+    blocks(oD + 9 * 10, C22[0], C22[1], C22[2]);
     // drilling (overwrites, as the reference)
     oD[9 * 5 + 8] = drill;   // D(5,5): block (1,1) entry (2,2)
     oD[9 * 15 + 8] = drill;  // D(11,11): block (3,3) entry (2,2)
     m1.z = drill * k.k1.z;
     m2.z = drill * k.k2.z;
+    sr.n1 = n1;
+    sr.n2 = n2;
+    sr.m1 = m1;
+    sr.m2 = m2;
+}
+
+__device__ __forceinline__ void shell_gp_rest(const ShellKin &k, const ShellRes &sr, double *o)
+{
+    const v3<double> n1 = sr.n1, n2 = sr.n2, m1 = sr.m1, m2 = sr.m2;
     m3<double> Qt = tr3(k.QQ);
     m3<double> QtXi = mm3(Qt, k.Xi);
     m3<double> Z1 = skew3(k.z1), Z2 = skew3(k.z2);
@@ -322,128 +328,211 @@ __device__ __forceinline__ void shell_gp_record(const double *__restrict__ cst, 
     st3(o + L_G + 36, madd(Ga1, Ga2));
 }
 
+// An element's constants in LDS: dN coefficients NU1, NU2, NA1, NA2, NA by Gauss
+// point, T3, the Gauss weight.
+constexpr int CF_NA1 = 36, CF_NA2 = 45, CF_NA = 54, CF_T3 = 63, CF_W = 72, CF_N = 73, CF_LD = 73;
+static_assert(SC_NU2 == SC_NU1 + 18, "NU1 and NU2 follow one another");
+
+__device__ __forceinline__ m3<double> mzero()
+{
+    m3<double> r;
+#pragma unroll
+    for (int q = 0; q < 9; q++) r.a[q] = 0.0;
+    return r;
+}
+// x of one lane of each four (CTRL: quad_perm of four times the same lane)
+template <int CTRL> __device__ __forceinline__ double quad_get(double x)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// K_IJ of element e, rotated to global
+__device__ __forceinline__ void k_store(double *__restrict__ Kout, int e, int I, int J, const double *t3, const m3<double> &Kl)
+{
+    const m3<double> T3 = ld3(t3), K = mtm3(T3, mm3(Kl, T3));
+    double *Ke = Kout + (size_t)e * 729;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) Ke[(3 * I + i) * 27 + 3 * J + j] = K.a[3 * i + j];
+}
+
+// Bound by its products' LDS reads (9 or 18 a product of 27 multiply-adds): 338 elements
+// 28 us -> 9, 8,192 90 -> 40, since each wavefront runs one form of its phase and the
+// constants are read once.
 template <bool PRE>
 __global__ __launch_bounds__(SWG, PRE ? 3 : 1) void shell_element_kernel(
     int e0, int e1, size_t ld, const int *__restrict__ conn, const double *__restrict__ cst,
     const double *__restrict__ gps, const double *__restrict__ disp, double *__restrict__ Kout,
     double *__restrict__ fout, const double *__restrict__ pre)
 {
-    __shared__ double sm[SEPB * 3 * L_GP];
+    __shared__ double sm[SEPB * 3 * L_GP + SEPB * CF_LD];
     const int tid = threadIdx.x;
     const int ebase = e0 + blockIdx.x * SEPB;
 
-    // ---- phase 1 (or its records from shell_record_kernel) ----------------------
+    const int lane = tid & 63, wave = tid >> 6, nv = min(SEPB, e1 - ebase);
+
+    // ---- the elements' constants; phase 1 (or its records from shell_record_kernel) ----
+    double *cf = sm + SEPB * 3 * L_GP;
+    for (int t = tid; t < SEPB * CF_N; t += SWG) {
+        const int le = t % SEPB, c = t / SEPB;
+        const int src = c < CF_NA1   ? SC_NU1 + c  // (NU1 and NU2 follow one another)
+                        : c < CF_NA2 ? SC_NA1 + c - CF_NA1
+                        : c < CF_NA  ? SC_NA2 + c - CF_NA2
+                        : c < CF_T3  ? SC_NA + c - CF_NA
+                        : c < CF_W   ? SC_T3 + c - CF_T3
+                                     : SC_ALPHA1;
+        if (le < nv) cf[le * CF_LD + c] = cst[(size_t)src * ld + ebase + le];
+    }
     if constexpr (PRE) {
-        const int nv = min(SEPB, e1 - ebase);
         const double *src = pre + (size_t)ebase * 3 * L_M;
-        for (int t = tid; t < nv * 3 * L_M; t += SWG) sm[(t / L_M) * L_GP + t % L_M] = src[t];
+        constexpr int NL = (SEPB * 3 * L_M + SWG - 1) / SWG;
+        double v[NL];
+#pragma unroll
+        for (int i = 0; i < NL; i++) v[i] = src[min(tid + SWG * i, nv * 3 * L_M - 1)];
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const int t = tid + SWG * i;
+            if (t < nv * 3 * L_M) sm[(t / L_M) * L_GP + t % L_M] = v[i];
+        }
     } else if (tid < 3 * SEPB) {
         int le = tid / 3, gp = tid - 3 * (tid / 3);
         int e = ebase + le;
         double *o = sm + (le * 3 + gp) * L_GP;
-        if (e < e1) shell_gp_record(cst, gps, ld, e, gp, disp, conn, o + L_D, o);
+        if (e < e1) {
+            ShellKin k;
+            ShellRes sr;
+            shell_kin(cst, gps, ld, e, gp, disp, conn, k);
+            shell_gp_moduli(cst, ld, e, k, o + L_D, sr);
+            shell_gp_rest(k, sr, o);
+        }
     }
     __syncthreads();
 
     // ---- phase 2: M blocks ---------------------------------------------------
-    for (int t = tid; t < SEPB * 3 * 25; t += SWG) {
-        int le = t / 75, rem = t - 75 * le, gp = rem / 25, rs = rem - 25 * gp;
-        int R = rs / 5, S = rs - 5 * R;
-        int e = ebase + le;
-        if (e >= e1) continue;
-        double *o = sm + (le * 3 + gp) * L_GP;
-        m3<double> Mb;
-        if (R < 4 && S < 4) {
-            Mb = mtm3(ld3(o + L_P + 9 * R), mm3(ld3(o + L_D + 9 * (4 * R + S)), ld3(o + L_P + 9 * S)));
-        } else if (R < 4) {
-            m3<double> V = mm3(ld3(o + L_D + 9 * (4 * R)), ld3(o + L_W));
-#pragma unroll
-            for (int j = 1; j < 4; j++) V = madd(V, mm3(ld3(o + L_D + 9 * (4 * R + j)), ld3(o + L_W + 9 * j)));
-            Mb = mtm3(ld3(o + L_P + 9 * R), V);
-            Mb = madd(Mb, g_block(o, R, false));
-        } else if (S < 4) {
+    // (R, S), R, S < 4: three wavefronts, two products a lane, after which the first
+    // takes the (4, S); the fourth the (R, 4), whose W_R^T V_R add up to (4, 4).
+    // (One lane a block in order sent every wavefront through all four forms: 20
+    // products for (4, 4) alone, twice where 300 tasks meet 256 lanes.)
+    if (wave < 3) {
+        const int p = tid >> 4, R = (tid >> 2) & 3, S = tid & 3;
+        if (p < 3 * nv) {
+            double *o = sm + p * L_GP;
+            st3(o + L_M + 9 * (5 * R + S),
+                mtm3(ld3(o + L_P + 9 * R), mm3(ld3(o + L_D + 9 * (4 * R + S)), ld3(o + L_P + 9 * S))));
+        }
+        if (wave == 0 && (lane >> 2) < 3 * nv) {
+            double *o = sm + (lane >> 2) * L_GP;
             m3<double> V = mtm3(ld3(o + L_W), ld3(o + L_D + 9 * S));
 #pragma unroll
             for (int i = 1; i < 4; i++) V = madd(V, mtm3(ld3(o + L_W + 9 * i), ld3(o + L_D + 9 * (4 * i + S))));
-            Mb = mm3(V, ld3(o + L_P + 9 * S));
-            Mb = madd(Mb, g_block(o, S, true));
-        } else {
-            m3<double> acc;
-#pragma unroll
-            for (int q = 0; q < 9; q++) acc.a[q] = 0.0;
-            for (int i = 0; i < 4; i++) {
-                m3<double> V = mm3(ld3(o + L_D + 9 * (4 * i)), ld3(o + L_W));
-                for (int j = 1; j < 4; j++) V = madd(V, mm3(ld3(o + L_D + 9 * (4 * i + j)), ld3(o + L_W + 9 * j)));
-                acc = madd(acc, mtm3(ld3(o + L_W + 9 * i), V));
-            }
-            Mb = madd(acc, ld3(o + L_G + 36));
+            st3(o + L_M + 9 * (20 + S), madd(mm3(V, ld3(o + L_P + 9 * S)), g_block(o, S, true)));
         }
-        st3(o + L_M + 9 * rs, Mb);
+    } else if ((lane >> 2) < 3 * nv) {
+        const int R = lane & 3;
+        double *o = sm + (lane >> 2) * L_GP;
+        m3<double> V = mm3(ld3(o + L_D + 9 * (4 * R)), ld3(o + L_W));
+#pragma unroll
+        for (int j = 1; j < 4; j++) V = madd(V, mm3(ld3(o + L_D + 9 * (4 * R + j)), ld3(o + L_W + 9 * j)));
+        st3(o + L_M + 9 * (5 * R + 4), madd(mtm3(ld3(o + L_P + 9 * R), V), g_block(o, R, false)));
+        const m3<double> U = mtm3(ld3(o + L_W + 9 * R), V);
+        m3<double> acc;
+#pragma unroll
+        for (int q = 0; q < 9; q++)
+            acc.a[q] = ((quad_get<0x00>(U.a[q]) + quad_get<0x55>(U.a[q])) + quad_get<0xAA>(U.a[q])) + quad_get<0xFF>(U.a[q]);
+        if (R == 0) st3(o + L_M + 9 * 24, madd(acc, ld3(o + L_G + 36)));
     }
     __syncthreads();
 
-    // ---- phase 3: K_IJ -------------------------------------------------------
-    for (int t = tid; t < SEPB * 81; t += SWG) {
-        int le = t / 81, ij = t - 81 * le;
-        int I = ij / 9, J = ij - 9 * (ij / 9);
-        int e = ebase + le;
-        if (e >= e1) continue;
-        double w = cst[SC_ALPHA1 * ld + e];
-        m3<double> K;
+    // ---- phase 3: K_IJ, by the number of M blocks it takes (9, 6, 4 a Gauss point) --
+    if (wave == 0) {
+        const int le = lane / 9, I = (lane - 9 * le) / 3, J = lane % 3;
+        if (le < nv) {
+            m3<double> K = mzero();
+            for (int gp = 0; gp < 3; gp++) {
+                const double *M = sm + (le * 3 + gp) * L_GP + L_M, *c = cf + le * CF_LD + CF_NA1 + 3 * gp;
 #pragma unroll
-        for (int q = 0; q < 9; q++) K.a[q] = 0.0;
-        for (int gp = 0; gp < 3; gp++) {
-            const double *o = sm + (le * 3 + gp) * L_GP;
-            int RI[3], RJ[3];
-            double cI[3], cJ[3];
-            int nI = col_rows(cst, ld, e, gp, I, RI, cI);
-            int nJ = col_rows(cst, ld, e, gp, J, RJ, cJ);
-            for (int a = 0; a < nI; a++)
-                for (int b = 0; b < nJ; b++) acc3(K.a, w * cI[a] * cJ[b], ld3(o + L_M + 9 * (5 * RI[a] + RJ[b])));
-        }
-        m3<double> T3;
+                for (int a = 0; a < 3; a++)
 #pragma unroll
-        for (int q = 0; q < 9; q++) T3.a[q] = cst[(SC_T3 + q) * ld + e];
-        K = mtm3(T3, mm3(K, T3));
-        double *Ke = Kout + (size_t)e * 729;
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int j = 0; j < 3; j++) Ke[(3 * I + i) * 27 + 3 * J + j] = K.a[3 * i + j];
-    }
-
-    // ---- phase 4: internal force ---------------------------------------------
-    for (int t = tid; t < SEPB * 9; t += SWG) {
-        int le = t / 9, I = t - 9 * le;
-        int e = ebase + le;
-        if (e >= e1) continue;
-        double w = cst[SC_ALPHA1 * ld + e];
-        v3<double> f = mk3(0.0, 0.0, 0.0);
-        for (int gp = 0; gp < 3; gp++) {
-            const double *o = sm + (le * 3 + gp) * L_GP;
-            int RI[3];
-            double cI[3];
-            int nI = col_rows(cst, ld, e, gp, I, RI, cI);
-            for (int a = 0; a < nI; a++) {
-                const double *S = o + L_S + 3 * RI[a];
-                f = add3(f, scl3(w * cI[a], mk3(S[0], S[1], S[2])));
+                    for (int b = 0; b < 3; b++)
+                        acc3(K.a, cf[le * CF_LD + CF_W] * c[9 * a + I] * c[9 * b + J],
+                             ld3(M + 9 * (5 * (a == 2 ? 4 : 1 + 2 * a) + (b == 2 ? 4 : 1 + 2 * b))));
             }
+            k_store(Kout, ebase + le, 6 + I, 6 + J, cf + le * CF_LD + CF_T3, K);
         }
-        m3<double> T3;
+    } else if (wave < 3) {
+        // displacement I against rotation J (18 a element), then the other way round
+        for (int t = lane + 64 * (wave - 1); t < 36 * SEPB; t += 128) {
+            const int le = t / 36, x = t - 36 * le, d = (x % 18) / 3, r = x % 3;
+            const bool rows = x < 18;  // displacement rows
+            if (le >= nv) break;
+            m3<double> K = mzero();
+            const int sd = rows ? 45 : 9, sr = rows ? 9 : 45;  // strides of M by the displacement's and the rotation's row
+            for (int gp = 0; gp < 3; gp++) {
+                const double *M = sm + (le * 3 + gp) * L_GP + L_M, *cd = cf + le * CF_LD + 6 * gp + d,
+                             *cr = cf + le * CF_LD + CF_NA1 + 3 * gp + r;
 #pragma unroll
-        for (int q = 0; q < 9; q++) T3.a[q] = cst[(SC_T3 + q) * ld + e];
-        f = mtv(T3, f);
-        fout[(size_t)e * 27 + 3 * I + 0] = f.x;
-        fout[(size_t)e * 27 + 3 * I + 1] = f.y;
-        fout[(size_t)e * 27 + 3 * I + 2] = f.z;
+                for (int a = 0; a < 2; a++)
+#pragma unroll
+                    for (int b = 0; b < 3; b++)
+                        acc3(K.a, cf[le * CF_LD + CF_W] * cd[18 * a] * cr[9 * b],
+                             ld3(M + 2 * a * sd + (b == 2 ? 4 : 1 + 2 * b) * sr));
+            }
+            k_store(Kout, ebase + le, rows ? d : 6 + r, rows ? 6 + r : d, cf + le * CF_LD + CF_T3, K);
+        }
+        // ---- phase 4: internal force ----------------------------------------
+        if (wave == 2 && lane < 9 * nv) {
+            const int le = lane / 9, I = lane - 9 * le;
+            const double *c = cf + le * CF_LD;
+            const double w = c[CF_W];
+            v3<double> f = mk3(0.0, 0.0, 0.0);
+            for (int gp = 0; gp < 3; gp++) {
+                const double *S = sm + (le * 3 + gp) * L_GP + L_S;
+                auto add = [&](double x, int R) { f = add3(f, scl3(w * x, mk3(S[3 * R], S[3 * R + 1], S[3 * R + 2]))); };
+                if (I < 6) {
+                    add(c[6 * gp + I], 0);
+                    add(c[18 + 6 * gp + I], 2);
+                } else {
+                    add(c[CF_NA1 + 3 * gp + I - 6], 1);
+                    add(c[CF_NA2 + 3 * gp + I - 6], 3);
+                    add(c[CF_NA + 3 * gp + I - 6], 4);
+                }
+            }
+            f = mtv(ld3(c + CF_T3), f);
+            double *fo = fout + (size_t)(ebase + le) * 27 + 3 * I;
+            fo[0] = f.x;
+            fo[1] = f.y;
+            fo[2] = f.z;
+        }
+    } else {
+        for (int t = lane; t < 36 * SEPB; t += 64) {
+            const int le = t / 36, I = (t - 36 * le) / 6, J = t % 6;
+            if (le >= nv) break;
+            m3<double> K = mzero();
+            for (int gp = 0; gp < 3; gp++) {
+                const double *M = sm + (le * 3 + gp) * L_GP + L_M, *c = cf + le * CF_LD + 6 * gp;
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+                        acc3(K.a, cf[le * CF_LD + CF_W] * c[18 * a + I] * c[18 * b + J], ld3(M + 9 * (10 * a + 2 * b)));
+            }
+            k_store(Kout, ebase + le, I, J, cf + le * CF_LD + CF_T3, K);
+        }
     }
 }
 
-// Follower pressure (MountShellSpecialLoads), lane per (element, u-node a) over all
-// elements: the record out[(6 e + a) SPR ...] holds the unbalanced-force change P_a
-// (3) and the load stiffness rows of node a (3 x 18, global frame); zeros for an
-// element without pressure.  The assembly (by rows or by colour) adds them to
-// the element's own.
+// Follower pressure (MountShellSpecialLoads) of all elements, PE a workgroup: a lane
+// per (element, point) finds the surface's tangents and normal there, then a lane per
+// (element, u-nodes a, b) sums the points.  The record out[(6 e + a) SPR ...] holds
+// the unbalanced-force change P_a (3) and the load stiffness rows of node a (3 x 18,
+// global frame); zeros for an element without pressure.  The assembly (by rows or by
+// colour) adds them to the element's own.  A lane per (element, a) with all of it took
+// 18 us at 338 elements (its 6 x 6 products one after another), 26 us at 8,192; a lane
+// per (element, a, b) that finds the tangents itself 11 and 40 us; this one 9 and 25.
+constexpr int PE = 7;
+
 __global__ __launch_bounds__(256) void shell_pressure_record_kernel(
     int ns, size_t ld, const int *__restrict__ conn, const double *__restrict__ cst,
     const double *__restrict__ pc, const double *__restrict__ disp, const double *__restrict__ copy,
@@ -451,49 +540,67 @@ __global__ __launch_bounds__(256) void shell_pressure_record_kernel(
     const double *__restrict__ lrec, const double *__restrict__ tab_t, const double *__restrict__ tab_v, const double *__restrict__ tp,
     double *__restrict__ out)
 {
+    __shared__ double sp[PE * 6][31];  // t1, t2, n, |t1 x t2|, w4, p; N, N1, N2 of the six nodes
     const double time = *tp;  // load time, device-resident (a captured Newton step reads the current one)
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    int e = t / 6, a = t - 6 * (t / 6);
-    if (e >= ns) return;
-    double *o = out + (size_t)t * SPR;
-    int L = pload[e];
+    const int tid = threadIdx.x, e0 = blockIdx.x * PE;
+    const int le = tid / 36, ab = tid - 36 * le, a = ab / 6, b = ab - 6 * a, e = e0 + le;
+    const bool act = le < PE && e < ns;
+    const int L = act ? pload[e] : -1;
+    for (int t = tid; t < PE * 108; t += 256) {
+        const int c = t / PE, l = t - PE * c, f = c / 36, ga = c - 36 * f;
+        const int row = (f == 0 ? SP_N4U : f == 1 ? SP_N4U1 : SP_N4U2) + ga;
+        sp[6 * l + ga / 6][12 + 6 * f + ga % 6] = pc[(size_t)row * ld + min(e0 + l, ns - 1)];
+    }
+    if (tid < 6 * PE && e0 + tid / 6 < ns) {
+        const int eg = e0 + tid / 6, g = tid % 6, Lg = pload[eg];
+        if (Lg >= 0) {
+            const double *rec = lrec + (size_t)Lg * NL_REC;
+            const double p = gf_table_value(tab_t, tab_v, (int)rec[NL_TAB0], (int)rec[NL_TABN], time, 0);
+            v3<double> t1 = mk3(cst[(SC_T3 + 0) * ld + eg], cst[(SC_T3 + 1) * ld + eg], cst[(SC_T3 + 2) * ld + eg]);
+            v3<double> t2 = mk3(cst[(SC_T3 + 3) * ld + eg], cst[(SC_T3 + 4) * ld + eg], cst[(SC_T3 + 5) * ld + eg]);
+#pragma unroll
+            for (int c = 0; c < 6; c++) {
+                const size_t nd = 6 * (size_t)conn[c * ld + eg];
+                const double d1 = pc[(SP_N4U1 + 6 * g + c) * ld + eg], d2 = pc[(SP_N4U2 + 6 * g + c) * ld + eg];
+                const v3<double> pu = mk3((copy[nd] - copy0[nd]) + disp[nd], (copy[nd + 1] - copy0[nd + 1]) + disp[nd + 1],
+                                          (copy[nd + 2] - copy0[nd + 2]) + disp[nd + 2]);
+                t1 = add3(t1, scl3(d1, pu));
+                t2 = add3(t2, scl3(d2, pu));
+            }
+            const v3<double> cr = cross3(t1, t2);
+            const double ncr = sqrt(dot3(cr, cr));
+            const v3<double> n = scl3(1.0 / ncr, cr);
+            double *o = sp[tid];
+            o[0] = t1.x; o[1] = t1.y; o[2] = t1.z;
+            o[3] = t2.x; o[4] = t2.y; o[5] = t2.z;
+            o[6] = n.x; o[7] = n.y; o[8] = n.z;
+            o[9] = ncr;
+            o[10] = pc[(SP_W4 + g) * ld + eg];
+            o[11] = p;
+        }
+    }
+    __syncthreads();
+    if (!act) return;
+    double *o = out + ((size_t)6 * e + a) * SPR;
     if (L < 0) {
-        for (int q = 0; q < SPR; q++) o[q] = 0.0;
+        for (int q = b; q < SPR; q += 6) o[q] = 0.0;
         return;
     }
-    const double *rec = lrec + (size_t)L * NL_REC;
-    double p = gf_table_value(tab_t, tab_v, (int)rec[NL_TAB0], (int)rec[NL_TABN], time, 0);
-    int au = pflag[e];
-    double pu[18];
-    for (int b = 0; b < 6; b++) {
-        int nd = conn[b * ld + e];
-#pragma unroll
-        for (int k = 0; k < 3; k++) pu[3 * b + k] = (copy[6 * (size_t)nd + k] - copy0[6 * (size_t)nd + k]) + disp[6 * (size_t)nd + k];
-    }
-    v3<double> e1r = mk3(cst[(SC_T3 + 0) * ld + e], cst[(SC_T3 + 1) * ld + e], cst[(SC_T3 + 2) * ld + e]);
-    v3<double> e2r = mk3(cst[(SC_T3 + 3) * ld + e], cst[(SC_T3 + 4) * ld + e], cst[(SC_T3 + 5) * ld + e]);
-    double Kr[3][18];
-    for (int i = 0; i < 3; i++)
-        for (int j = 0; j < 18; j++) Kr[i][j] = 0.0;
+    const int au = pflag[e];
+    double Kr[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     v3<double> Pa = mk3(0.0, 0.0, 0.0);
+#pragma unroll 2
     for (int g = 0; g < 6; g++) {
-        v3<double> t1 = e1r, t2 = e2r;
-        for (int b = 0; b < 6; b++) {
-            double c1 = pc[(SP_N4U1 + 6 * g + b) * ld + e], c2 = pc[(SP_N4U2 + 6 * g + b) * ld + e];
-            t1 = add3(t1, scl3(c1, mk3(pu[3 * b], pu[3 * b + 1], pu[3 * b + 2])));
-            t2 = add3(t2, scl3(c2, mk3(pu[3 * b], pu[3 * b + 1], pu[3 * b + 2])));
-        }
-        v3<double> cr = cross3(t1, t2);
-        double ncr = sqrt(dot3(cr, cr));
-        v3<double> n = scl3(1.0 / ncr, cr);
-        double w4 = pc[(SP_W4 + g) * ld + e];
-        double Na = pc[(SP_N4U + 6 * g + a) * ld + e];
-        double jac = au ? ncr : 1.0;
+        const double *q = sp[6 * le + g];
+        const v3<double> t1 = mk3(q[0], q[1], q[2]), t2 = mk3(q[3], q[4], q[5]), n = mk3(q[6], q[7], q[8]);
+        const double ncr = q[9], w4 = q[10], p = q[11], Na = q[12 + a], c1 = q[18 + b], c2 = q[24 + b];
+        const double jac = au ? ncr : 1.0;
         // unbalanced force change: P -= w4 jac N4^T q with q = -p n
         Pa = add3(Pa, scl3(w4 * jac * Na * p, n));
-        m3<double> S1 = skew3(t1), S2 = skew3(t2);
-        m3<double> Pm;
+        const m3<double> S1 = skew3(t1), S2 = skew3(t2);
+        m3<double> B = msub(mscl(c2, S1), mscl(c1, S2));
         if (!au) {
+            m3<double> Pm;
 #pragma unroll
             for (int i = 0; i < 3; i++)
 #pragma unroll
@@ -501,50 +608,68 @@ __global__ __launch_bounds__(256) void shell_pressure_record_kernel(
                     double ni = i == 0 ? n.x : (i == 1 ? n.y : n.z), nj = j == 0 ? n.x : (j == 1 ? n.y : n.z);
                     Pm.a[3 * i + j] = ((i == j ? 1.0 : 0.0) - ni * nj) / ncr;
                 }
+            B = mm3(Pm, B);
         }
-        double s = w4 * 1.0 * p * Na;
-        for (int b = 0; b < 6; b++) {
-            double c1 = pc[(SP_N4U1 + 6 * g + b) * ld + e], c2 = pc[(SP_N4U2 + 6 * g + b) * ld + e];
-            m3<double> B = msub(mscl(c2, S1), mscl(c1, S2));
-            if (!au) B = mm3(Pm, B);
+        const double s = w4 * 1.0 * p * Na;
 #pragma unroll
-            for (int i = 0; i < 3; i++)
-#pragma unroll
-                for (int j = 0; j < 3; j++) Kr[i][3 * b + j] += s * B.a[3 * i + j];
-        }
+        for (int i = 0; i < 9; i++) Kr[i] += s * B.a[i];
     }
     // the element's unbalanced force grows by Pa (the residual takes its negative)
-    o[0] = Pa.x;
-    o[1] = Pa.y;
-    o[2] = Pa.z;
+    if (b < 3) o[b] = b == 0 ? Pa.x : b == 1 ? Pa.y : Pa.z;
+#pragma unroll
     for (int i = 0; i < 3; i++)
-        for (int j = 0; j < 18; j++) o[3 + 18 * i + j] = Kr[i][j];
+#pragma unroll
+        for (int j = 0; j < 3; j++) o[3 + 18 * i + 3 * b + j] = Kr[3 * i + j];
 }
 
 // Phase 1 of every element's Gauss points in one launch: lane per (element, gp),
-// its D blocks accumulated in LDS (74 KB per 64 lanes, two workgroups per CU;
-// a lane's stride of 145 entries keeps a wavefront's accesses off shared banks)
-// and copied out record by record, the write-once rest stored directly.  The
-// element kernel reads the records instead of recomputing phase 1 on 12 lanes
-// per workgroup.
-constexpr int REC_LANES = 64, REC_DS = 145;
-__global__ __launch_bounds__(REC_LANES) void shell_record_kernel(int ns, size_t ld, const int *__restrict__ conn,
-                                                                  const double *__restrict__ cst,
-                                                                  const double *__restrict__ gps,
-                                                                  const double *__restrict__ disp, double *__restrict__ rec)
+// NP points a wavefront.  A wavefront's instructions bound it (stores of 8 bytes in 64
+// lines, and sums in LDS, took half of 26 us at 338 elements, 37 at 8,192; now 12 and
+// 22).  Both parts of the record pass through LDS and are copied
+// out by all 64 lanes, in rows (a lane's stride is odd: a wavefront's accesses stay
+// off shared banks).  The element kernel reads the records instead of recomputing
+// phase 1 on 12 lanes per workgroup.
+constexpr int REC_DS = 145;
+
+__device__ __forceinline__ void record_rows(double *dst, const double *src, int stride, int width, int nt)
 {
-    __shared__ double sD[REC_LANES * REC_DS];
-    const int t0 = blockIdx.x * REC_LANES, t = t0 + threadIdx.x;
-    const int nt = min(REC_LANES, 3 * ns - t0);
-    if ((int)threadIdx.x < nt) {
-        const int e = t / 3, gp = t - 3 * (t / 3);
-        shell_gp_record(cst, gps, ld, e, gp, disp, conn, sD + threadIdx.x * REC_DS, rec + (size_t)t * L_M);
+    int i = threadIdx.x, r = 0;  // (width > 64: an entry is at most one row further)
+    const int n = nt * width;
+#pragma unroll 4
+    for (int q = threadIdx.x; q < n; q += 64) {
+        dst[(size_t)r * L_M + i] = src[r * stride + i];
+        i += 64;
+        if (i >= width) {
+            i -= width;
+            r++;
+        }
+    }
+}
+
+template <int NP>
+__global__ __launch_bounds__(64) void shell_record_kernel(int ns, size_t ld, const int *__restrict__ conn,
+                                                          const double *__restrict__ cst,
+                                                          const double *__restrict__ gps,
+                                                          const double *__restrict__ disp, double *__restrict__ rec)
+{
+    __shared__ double sD[NP * REC_DS];
+    const int t0 = blockIdx.x * NP, t = t0 + threadIdx.x;
+    const int nt = min(NP, 3 * ns - t0);
+    const bool act = (int)threadIdx.x < nt;
+    const int e = t / 3, gp = t - 3 * (t / 3);
+    double *own = sD + threadIdx.x * REC_DS, *out = rec + (size_t)t0 * L_M;
+    ShellKin k;
+    ShellRes sr;
+    if (act) {
+        shell_kin(cst, gps, ld, e, gp, disp, conn, k);
+        shell_gp_moduli(cst, ld, e, k, own, sr);
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < nt * 144; q += REC_LANES) {
-        const int r = q / 144, i = q - 144 * r;
-        rec[(size_t)(t0 + r) * L_M + L_D + i] = sD[r * REC_DS + i];
-    }
+    record_rows(out + L_D, sD, REC_DS, L_P - L_D, nt);
+    __syncthreads();
+    if (act) shell_gp_rest(k, sr, own - L_P);
+    __syncthreads();
+    record_rows(out + L_P, sD, REC_DS, L_M - L_P, nt);
 }
 
 __global__ __launch_bounds__(256) void shell_commit_kernel(int ns, size_t ld, const int *__restrict__ conn,
@@ -972,11 +1097,14 @@ int gf_shell_assemble(gf_model *m, const double *lfp, const double *tp)
     int launches = 0;
     if (m->ns == 0) return 0;
     // phase 1 of every element and the pressure terms
-    hipLaunchKernelGGL(shell_record_kernel, dim3((3 * m->ns + REC_LANES - 1) / REC_LANES), dim3(REC_LANES), 0,
-                       m->stream, m->ns, ld, m->d_sconn, m->d_sconst, m->d_sgp, m->d_disp, m->d_shell_rec);
+    // (a wavefront's time hardly depends on its points but for the copy: as few as leave one wavefront a SIMD)
+    const int np = 3 * m->ns, per = np <= 16 * 1024 ? 16 : np <= 32 * 1024 ? 32 : 64;
+    hipLaunchKernelGGL(per == 16 ? shell_record_kernel<16> : per == 32 ? shell_record_kernel<32> : shell_record_kernel<64>,
+                       dim3((np + per - 1) / per), dim3(64), 0, m->stream, m->ns, ld, m->d_sconn, m->d_sconst, m->d_sgp,
+                       m->d_disp, m->d_shell_rec);
     launches++;
     if (m->any_pressure) {
-        hipLaunchKernelGGL(shell_pressure_record_kernel, dim3((6 * m->ns + 255) / 256), dim3(256), 0, m->stream,
+        hipLaunchKernelGGL(shell_pressure_record_kernel, dim3((m->ns + PE - 1) / PE), dim3(256), 0, m->stream,
                            m->ns, ld, m->d_sconn, m->d_sconst, m->d_spconst, m->d_disp, m->d_copy, m->d_copy0,
                            m->d_spload, m->d_spflag, m->d_lrec, m->d_tab_t, m->d_tab_v, tp, m->d_shell_prec);
         launches++;
