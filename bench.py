@@ -182,7 +182,7 @@ KERNEL_NAMES = {"btd_level": "cr_reduce_kernel (per halving of the rows)", "btd_
                 "band_sweep": "band_batch_apply_kernel + band_couple_kernel",
                 "beam_assemble": "beam_assemble_kernel<0>", "shell_assemble": "shell_element_kernel",
                 "front_step": "front_step_kernel", "front_assemble": "front_assemble_kernel",
-                "front_solve": "front_fwd_own/fwd_upd/bwd_upd/bwd_own_kernel"}
+                "front_solve": "front_fwd_own/fwd_upd/bwd/bwd_upd/bwd_own_kernel"}
 
 
 def kernel_work(cls, info):

@@ -33,7 +33,8 @@
 //             its update vector  c = sum_children c_child - L(t, own) y.
 //   backward  per level from the root: x_own = y - U(own, update) x_update
 //             (row tiles in parallel, x_update read from the ancestors' rows of
-//             x), then the own-block back substitution and the scatter of x.
+//             x), then the own-block back substitution and the scatter of x; in
+//             one launch where the plan finds the rows few.
 #include "gf_tile.h"
 
 #include <algorithm>
@@ -41,7 +42,7 @@
 
 namespace {
 
-constexpr int KMAX = 1024;  // largest own block (rows in LDS of the solve); the plan splits larger supernodes
+constexpr int KMAX = GF_FRONT_KMAX;  // largest own block (rows in LDS of the solve); the plan splits larger supernodes
 
 struct FrontTab {
     const gf_front_dev *fr;
@@ -711,6 +712,104 @@ __global__ __launch_bounds__(256) void front_bwd_own_kernel(FrontTab t, int f0, 
     for (int i = tid; i < F.k; i += 256) x[rows[i]] = y[i];
 }
 
+// Next tile of the upper block rows in the order of use: row p's columns p + 1 .. mb - 1,
+// p from the last down; past the last, that one again.
+template <typename T>
+__device__ __forceinline__ void bwd_fetch(RowTile<T> &a, const T *U, unsigned ld, int mb, int &p, int &j)
+{
+    a.load(U + (size_t)(NB * p * ld) + NB * j, ld);
+    const bool end = j + 1 >= mb;
+    j = !end ? j + 1 : p > 0 ? p : j;
+    p = end && p > 0 ? p - 1 : p;
+}
+// Row's end: y -= sums, which are cleared.
+__device__ __forceinline__ void bwd_row(double (&acc)[8], double *y)
+{
+    const double s = tile_sum(acc);
+    if ((threadIdx.x & 3) == 0) y[tile_row()] -= s;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc[k] = 0.0;
+}
+// The last own row's end (see front_bwd_upd_kernel); w: 64 doubles of LDS.
+template <typename T>
+__device__ __forceinline__ void bwd_last(double (&acc)[8], const RowTile<T> &e, double *y, double *w, int raw)
+{
+    const int r = tile_row();
+    const bool lead = (threadIdx.x & 3) == 0;
+    const double part = tile_sum(acc), y0 = lead ? y[r] : 0.0;
+    if (lead) w[r] = raw ? y0 - part : part;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc[k] = 0.0;
+    e.dot(acc, w);
+    const double s = tile_sum(acc);
+    if (lead) y[r] = raw ? s : y0 - s;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc[k] = 0.0;
+}
+
+// The two above in one, a workgroup a front, for the levels where the plan says so
+// (bwd_one): x_p = z_p - U(p, p+1 ..) (x_own | x_update), p from the last row up, over
+// one vector in LDS.  Three tiles are in flight, without a move or a branch between
+// a load and its use (past the last tile the last one is loaded again).  Bound by its
+// launch and the chain front record, rows, x: 7 us for a level of small fronts in
+// place of 5.1 + 4.6, a root of 9 own blocks 25.6 us where one tile in flight took 28.7.
+template <typename T>
+__global__ __launch_bounds__(256) void front_bwd_kernel(FrontTab t, int f0, const T *Fb, const T *Eb, const double *Vb,
+                                                        double *x, int raw_last)
+{
+    __shared__ alignas(16) double v[KMAX];
+    __shared__ alignas(16) double w[NB];
+    const gf_front_dev F = t.fr[f0 + blockIdx.x];
+    const int kp = NB * F.kb, tid = threadIdx.x;
+    const int *rows = t.rows + F.rows;
+    const unsigned ld = F.mp;
+    const T *U = Fb + F.F;
+    const bool upd = F.mb > F.kb;
+    int p = upd ? F.kb - 1 : F.kb - 2, j = p + 1;  // next tile to use
+    int lp = max(p, 0), lj = min(lp + 1, F.mb - 1);    // next tile to load
+    RowTile<T> a, b, c, e;
+    bwd_fetch(a, U, ld, F.mb, lp, lj);
+    e.load(Eb + F.E + (size_t)((F.kb - 1) * NB * NB), NB);
+    bwd_fetch(b, U, ld, F.mb, lp, lj);
+    bwd_fetch(c, U, ld, F.mb, lp, lj);
+    for (int i = tid; i < F.mp; i += 256) {
+        const int o = i < kp ? 0 : rows[i];
+        v[i] = i < kp ? Vb[F.V + i] : o >= 0 ? x[o] : 0.0;
+    }
+    __syncthreads();
+    double acc[8] = {};
+    if (!upd && raw_last) bwd_last(acc, e, v + kp - NB, w, raw_last);
+    while (p >= 0) {
+        a.dot(acc, v + NB * j);
+        bwd_fetch(a, U, ld, F.mb, lp, lj);
+        if (++j == F.mb) {
+            if (p == F.kb - 1) bwd_last(acc, e, v + kp - NB, w, raw_last);
+            else bwd_row(acc, v + NB * p);
+            j = p--;
+        }
+        if (p < 0) break;
+        b.dot(acc, v + NB * j);
+        bwd_fetch(b, U, ld, F.mb, lp, lj);
+        if (++j == F.mb) {
+            if (p == F.kb - 1) bwd_last(acc, e, v + kp - NB, w, raw_last);
+            else bwd_row(acc, v + NB * p);
+            j = p--;
+        }
+        if (p < 0) break;
+        c.dot(acc, v + NB * j);
+        bwd_fetch(c, U, ld, F.mb, lp, lj);
+        if (++j == F.mb) {
+            if (p == F.kb - 1) bwd_last(acc, e, v + kp - NB, w, raw_last);
+            else bwd_row(acc, v + NB * p);
+            j = p--;
+        }
+    }
+    for (int i = tid; i < F.k; i += 256) x[rows[i]] = v[i];
+}
+
 FrontTab tab_of(const gf_fronts &fp)
 {
     FrontTab t;
@@ -794,6 +893,14 @@ int front_solve_t(const gf_fronts &fp, const T *F, const T *E, const double *rhs
     for (int l = fp.n_level - 1; l >= 0; l--) {
         const int nf = fp.lev_off[l + 1] - fp.lev_off[l];
         int pr;
+        if (fp.bwd_one[l]) {
+            pr = gf_probe_begin(s, GF_KC_FRONT_SOLVE);
+            hipLaunchKernelGGL(front_bwd_kernel<T>, dim3(nf), dim3(256), 0, s, t, fp.lev_off[l], F, E, (const double *)V, x,
+                               carried ? 1 : 0);
+            gf_probe_end(s, pr, pr >= 0 ? panel_bytes(l) + own_bytes(l, false) : 0.0);
+            launches++;
+            continue;
+        }
         if (fp.bupd_count[l] > 0) {
             pr = gf_probe_begin(s, GF_KC_FRONT_SOLVE);
             hipLaunchKernelGGL(front_bwd_upd_kernel<T>, dim3(fp.bupd_count[l]), dim3(256), 0, s, t, fp.bupd_first[l], F,

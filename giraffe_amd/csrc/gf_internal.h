@@ -292,6 +292,8 @@ struct gf_front_dev {
     int ch0, ch1;       // children: entries [ch0, ch1) of the child lists
     int pad;
 };
+constexpr int GF_FRONT_KMAX = 1024;  // rows of a front that the solve kernels hold in LDS
+
 struct gf_fronts {
     int n_front = 0, n_level = 0, max_k = 0;
     std::vector<gf_front_dev> fr;
@@ -307,6 +309,7 @@ struct gf_fronts {
     std::vector<int> asm_first, asm_count;    // per level: assembly tiles
     std::vector<int> fupd_first, fupd_count;  // per level: forward update row tiles (front, tile row)
     std::vector<int> bupd_first, bupd_count;  // per level: backward own row tiles with an update part
+    std::vector<char> bwd_one;         // per level: backward in one launch, a workgroup a front
     std::vector<double> step_flops;    // algorithmic flops of each factor launch
     std::vector<int> orig;             // tangent entries of the assembly tiles: position in the tile, band row, band column
     std::vector<int> asm_orig;         // per work item (2 ints): first entry of its tile in orig, count

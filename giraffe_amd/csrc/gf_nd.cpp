@@ -371,6 +371,14 @@ int gf_nd_plan(gf_fronts &fp, const gf_model_desc *d, const std::vector<int> &do
                 for (int p = 0; p < fp.fr[f].kb; p++) fp.items.insert(fp.items.end(), {f, p, 0, 0});
         fp.bupd_first.push_back(b0);
         fp.bupd_count.push_back((int)fp.items.size() / 4 - b0);
+        // One workgroup a front instead of one a row tile, then one a front: a launch
+        // less (4.6 us), for (kb - 1) times the update tiles in a row in place of side
+        // by side (0.5 us each: 8 fronts of 3 x 6 blocks take 12.6 us this way and 7.4 +
+        // 4.7 the other, 8 of 1 x 3 8.0 and 5.9 + 4.7).
+        bool one = true;
+        for (int f = fp.lev_off[l]; f < fp.lev_off[l + 1]; f++)
+            one = one && fp.fr[f].mp <= GF_FRONT_KMAX && (fp.fr[f].kb - 1) * (fp.fr[f].mb - fp.fr[f].kb) <= 8;
+        fp.bwd_one.push_back(one);
     }
     return GF_OK;
 }
@@ -385,7 +393,7 @@ int gf_front_factor_launches(const gf_fronts &fp)
 int gf_front_solve_launches(const gf_fronts &fp)
 {
     int n = 0;
-    for (int l = 0; l < fp.n_level; l++) n += 2 + (fp.fupd_count[l] > 0) + (fp.bupd_count[l] > 0);
+    for (int l = 0; l < fp.n_level; l++) n += 2 + (fp.fupd_count[l] > 0) + (fp.bupd_count[l] > 0 && !fp.bwd_one[l]);
     return n;
 }
 
