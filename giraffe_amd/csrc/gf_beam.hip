@@ -26,6 +26,7 @@
 // so one launch per colour scatters without atomics and deterministically.
 #include "gf_internal.h"
 #include "gf_device.h"
+#include "gf_loads.h"
 
 namespace {
 
@@ -100,9 +101,20 @@ __global__ __launch_bounds__(SPLIT ? 2 * WG : WG) void beam_assemble_kernel(
     const double *__restrict__ gps, const double *__restrict__ disp, const int *__restrict__ dof,
     gf_gmat gm, double *__restrict__ r, const double *__restrict__ lfp, double gx, double gy, double gz,
     double *__restrict__ Kout, double *__restrict__ fout, const double *__restrict__ buoy,
-    const double *__restrict__ copy, double sx, double sy, double sz)
+    const double *__restrict__ copy, double sx, double sy, double sz, int nwork, gf_nodal loads)
 {
     __shared__ double sm[EPB * 2 * LDS_GP];
+    if (MODE == 0 && (int)blockIdx.x >= nwork) {  // (uniform)
+        // the nodal loads, beside the elements: a chain of its own, 7 to 10 us as a launch
+        const int k = ((int)blockIdx.x - nwork) * (int)blockDim.x + (int)threadIdx.x;
+        if (k >= loads.n) return;
+        double q[GF_NODAL_OUT];
+        gf_nodal_item(loads, k, q);
+        double *o = loads.out + (size_t)GF_NODAL_OUT * k;
+#pragma unroll
+        for (int i = 0; i < GF_NODAL_OUT; i++) o[i] = q[i];
+        return;
+    }
     const int tid = threadIdx.x & 63;
     const bool w0 = !SPLIT || threadIdx.x < 64, w1 = !SPLIT || threadIdx.x >= 64;  // phase 2; phases 1 and 3
     const int ebase = e0 + blockIdx.x * EPB;
@@ -461,7 +473,7 @@ void gf_beam_host_const(const double *x, const double *cs, const double *prop, i
     }
 }
 
-int gf_beam_assemble(gf_model *m, const double *lfp)
+int gf_beam_assemble(gf_model *m, const double *lfp, const double *tp)
 {
     const size_t ld = (size_t)m->nb;
     int ncol = (int)m->beam_color_off.size() - 1;
@@ -469,15 +481,16 @@ int gf_beam_assemble(gf_model *m, const double *lfp)
     for (int c = 0; c < ncol; c++) {
         int e0 = m->beam_color_off[c], e1 = m->beam_color_off[c + 1];
         if (e1 <= e0) continue;
-        launches++;
         int grid = (e1 - e0 + EPB - 1) / EPB;
+        const gf_nodal loads = launches == 0 && m->d_ln_out ? gf_nodal_of(m, tp) : gf_nodal();
+        launches++;
         const int pr = gf_probe_begin(m->stream, GF_KC_BEAM_ASSEMBLE);
         auto launch = [&](auto kernel, int threads) {
-            hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, m->stream, e0, e1, ld, m->d_bconn, m->d_bconst,
+            hipLaunchKernelGGL(kernel, dim3(grid + (loads.n + threads - 1) / threads), dim3(threads), 0, m->stream, e0, e1, ld, m->d_bconn, m->d_bconst,
                                m->d_bgp, m->d_disp, m->d_dof, gf_model_gmat(m), m->d_r, lfp, m->gravity[0],
                                m->gravity[1], m->gravity[2], (double *)nullptr, (double *)nullptr,
                                (const double *)m->d_bbuoy, (const double *)m->d_copy, m->ocean_surface[0],
-                               m->ocean_surface[1], m->ocean_surface[2]);
+                               m->ocean_surface[1], m->ocean_surface[2], grid, loads);
         };
         if (grid <= 512) launch(beam_assemble_kernel<0, true>, 2 * WG);
         else launch(beam_assemble_kernel<0, false>, WG);
@@ -542,7 +555,7 @@ int gf_beam_eval_device(int count, const double *x, const double *cs, const doub
     hipLaunchKernelGGL((beam_assemble_kernel<1, false>), dim3(grid), dim3(WG), 0, s, 0, count, ld, d_conn, d_cst, d_gps,
                        d_disp, (const int *)nullptr, none, (double *)nullptr, (const double *)nullptr, 0.0, 0.0, 0.0, d_K,
                        d_f,
-                       (const double *)nullptr, (const double *)nullptr, 0.0, 0.0, 0.0);
+                       (const double *)nullptr, (const double *)nullptr, 0.0, 0.0, 0.0, grid, gf_nodal());
     GF_HIP(hipGetLastError());
     GF_HIP(hipMemcpyAsync(K_out, d_K, sizeof(double) * 324 * ld, hipMemcpyDeviceToHost, s));
     GF_HIP(hipMemcpyAsync(f_out, d_f, sizeof(double) * 18 * ld, hipMemcpyDeviceToHost, s));

@@ -463,6 +463,9 @@ struct gf_model {
     // device: nodal loads
     int n_load_nodes = 0;
     int *d_ln_node = nullptr, *d_ln_off = nullptr, *d_ln_ids = nullptr;
+    // models with beams: the loads' contributions (gf_loads.h), and each row's entry of them or -1
+    double *d_ln_out = nullptr;
+    int *d_row_load = nullptr;
     double *d_lrec = nullptr;       // [nl][NL_REC]
     double *d_tab_t = nullptr, *d_tab_v = nullptr;
 
@@ -556,7 +559,7 @@ int gf_launch_clear_csr(hipStream_t s, double *a, size_t na, double *c, size_t n
 // p[0] = a, p[1] = b (a kernel, so it can sit in a captured graph)
 int gf_launch_set2(hipStream_t s, double *p, double a, double b);
 // Returns the number of kernel launches issued (>= 0) or a negative status.
-int gf_beam_assemble(gf_model *m, const double *lfp);
+int gf_beam_assemble(gf_model *m, const double *lfp, const double *tp);
 int gf_beam_commit(gf_model *m);
 int gf_shell_assemble(gf_model *m, const double *lfp, const double *tp);  // elements + follower pressure
 int gf_shell_eval_device(int count, const double *x, const double *prop, const double *d, const double *gp,

@@ -170,7 +170,7 @@ static void release(gf_model *m)
                     m->d_scal, m->d_copy0, m->d_bgp0, m->d_sconn, m->d_sconst, m->d_spconst, m->d_sgp,
                     m->d_sgp0, m->d_spload, m->d_spflag, m->d_band, m->d_swork, m->d_band_inv, m->d_bbuoy,
                     m->d_front, m->d_front_e, m->d_front_v, m->d_csr_ptr, m->d_csr_col, m->d_shell_rec,
-                    m->d_shell_prec, m->d_shell_K, m->d_shell_f, m->d_sg_ptr, m->d_sg_list, m->d_sg_pos};
+                    m->d_shell_prec, m->d_shell_K, m->d_shell_f, m->d_sg_ptr, m->d_sg_list, m->d_sg_pos, m->d_ln_out, m->d_row_load};
     for (void *b : bufs) gf_pool_free(b);
     gf_front_free(m->fronts);
     if (m->h_scal) gf_pinned_free(m->h_scal);
@@ -500,6 +500,7 @@ static size_t footprint(const gf_model_desc *d, const gf_model *m, int precision
     size_t items = d->n_loads ? (size_t)d->load_set_off[d->n_loads] : 0;
     size_t rows = d->n_loads ? (size_t)d->load_tab_off[d->n_loads] : 0;
     b += (size_t)d->n_loads * NL_REC * 8 + items * 12 + rows * 7 * 8;         // loads and tables
+    if (nb > 0 && items > 0) b += items * 24 * 8 + npad * 4;                  // their contributions
     b += 3 * npad * 8 + 256;                                                   // r, x, work, scalars
     size_t tangent;
     if (m->layout == GM_BTD) {
@@ -743,6 +744,18 @@ static int create(const gf_model_desc *d, const gf_options *opt, gf_model *m)
         GF_TRY(dalloc(&m->d_tab_t, (size_t)rows));
         GF_TRY(dalloc(&m->d_tab_v, 6 * (size_t)rows));
         GF_TRY(upload(m, m->d_ln_node, ln_node.data(), ln_node.size()));
+        std::vector<int> row_load;
+        if (nb > 0 && m->n_load_nodes > 0) {
+            row_load.assign((size_t)m->npad, -1);
+            for (int k = 0; k < m->n_load_nodes; k++)
+                for (int c = 0; c < 6; c++) {
+                    const int r = m->dof[6 * (size_t)ln_node[k] + c];
+                    if (r >= 0) row_load[r] = 6 * k + c;
+                }
+            GF_TRY(dalloc(&m->d_ln_out, 24 * ln_node.size()));
+            GF_TRY(dalloc(&m->d_row_load, row_load.size()));
+            GF_TRY(upload(m, m->d_row_load, row_load.data(), row_load.size()));
+        }
         GF_TRY(upload(m, m->d_ln_off, ln_off.data(), ln_off.size()));
         GF_TRY(upload(m, m->d_ln_ids, ln_ids.data(), ln_ids.size()));
         GF_TRY(upload(m, m->d_lrec, lrec.data(), lrec.size()));
@@ -1108,9 +1121,10 @@ int gf_assemble_enqueue(gf_model *m, bool cleared)
     // load time and gravity ramp factor from the scalar block (set by gf_begin_step)
     const double *tp = m->d_scal + GF_SCAL_TIME, *lfp = m->d_scal + GF_SCAL_LF;
     // (the assembly by rows writes where the others add, so it comes first)
-    if (!m->shell_gather) GF_TRY(gf_nodal_loads(m, tp));
+    // (nor where the first beam launch forms them and the scan adds them)
+    if (!m->shell_gather && !m->d_ln_out) GF_TRY(gf_nodal_loads(m, tp));
     tick(m, GF_PH_ASSEMBLE, true);
-    GF_TRYN(nl_beam, gf_beam_assemble(m, lfp));
+    GF_TRYN(nl_beam, gf_beam_assemble(m, lfp, tp));
     GF_TRYN(nl_shell, gf_shell_assemble(m, lfp, tp));
     tick(m, GF_PH_ASSEMBLE, false);
     if (m->shell_gather) GF_TRY(gf_nodal_loads(m, tp));

@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include "gf_device.h"
+#include "gf_loads.h"
 
 namespace {
 
@@ -70,88 +71,28 @@ __global__ void fill_u32_kernel(unsigned *p, size_t n)
 }
 
 
-// One thread per loaded node: all loads on that node, in load order.
-__global__ __launch_bounds__(128) void nodal_loads_kernel(int n_ln, const int *__restrict__ ln_node, const int *__restrict__ ln_off,
-                                   const int *__restrict__ ln_ids, const double *__restrict__ rec,
-                                   const double *__restrict__ tab_t, const double *__restrict__ tab_v,
-                                   const double *__restrict__ disp, const double *__restrict__ copy,
-                                   const int *__restrict__ dof, gf_gmat gm, double *r, const double *__restrict__ tp)
+// One thread per loaded node.  (Models with beams take them with the first beam
+// launch and the scan instead.)
+__global__ __launch_bounds__(128) void nodal_loads_kernel(gf_nodal L, const int *__restrict__ dof, gf_gmat gm, double *r)
 {
-    const double t = *tp;  // load time, device-resident (a captured Newton step reads the current one)
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n_ln) return;
-    int node = ln_node[k];
-    int R[6];
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= L.n) return;
+    double q[GF_NODAL_OUT], q6[6], V18[18];
+    gf_nodal_item(L, k, q);
+    int R[6], R18[18], C18[18];
 #pragma unroll
-    for (int i = 0; i < 6; i++) R[i] = dof[6 * node + i];
-    v3<double> alpha = mk3(disp[6 * node + 3], disp[6 * node + 4], disp[6 * node + 5]);
-    for (int q = ln_off[k]; q < ln_off[k + 1]; q++) {
-        const double *L = rec + (size_t)ln_ids[q] * NL_REC;
-        int kind = (int)L[NL_KIND];
-        m3<double> CS;
-#pragma unroll
-        for (int i = 0; i < 9; i++) CS.a[i] = L[NL_CS + i];
-        int r0 = (int)L[NL_TAB0], nt = (int)L[NL_TABN];
-        double tv6[6];
-        gf_table_values6(tab_t, tab_v, r0, nt, t, tv6);
-        v3<double> f = mk3(L[NL_MULT + 0] * tv6[0], L[NL_MULT + 1] * tv6[1], L[NL_MULT + 2] * tv6[2]);
-        v3<double> mo = mk3(L[NL_MULT + 3] * tv6[3], L[NL_MULT + 4] * tv6[4], L[NL_MULT + 5] * tv6[5]);
-        if (kind == GF_LOAD_NODAL) {
-            // dead force + pseudo-moment Xi^T m with stiffness -V(alpha, Xi^T m)
-            f = mtv(CS, f);
-            mo = mtv(CS, mo);
-            m3<double> Q, Xi;
-            double g;
-            rodrigues(alpha, Q, Xi, g);
-            mo = mtv(Xi, mo);
-            m3<double> S = opV(alpha, mo);
-            const double q6[6] = {f.x, f.y, f.z, mo.x, mo.y, mo.z};
-            vec_add_n<6>(r, R, q6);
-            int R9[9], C9[9];
-            double V9[9];
-#pragma unroll
-            for (int i = 0; i < 3; i++)
-#pragma unroll
-                for (int j = 0; j < 3; j++) {
-                    R9[3 * i + j] = R[3 + i];
-                    C9[3 * i + j] = R[3 + j];
-                    V9[3 * i + j] = -S.a[3 * i + j];
-                }
-            gm_add_n<9>(gm, R9, C9, V9);
-        } else if (kind == GF_LOAD_NODAL_FOLLOWER) {
-            v3<double> ai = mk3(copy[6 * node + 3], copy[6 * node + 4], copy[6 * node + 5]);
-            m3<double> Qi, Xii, Q, Xi;
-            double gi, g;
-            rodrigues(ai, Qi, Xii, gi);
-            Qi = mm3(Qi, tr3(CS));
-            rodrigues(alpha, Q, Xi, g);
-            v3<double> fip = mv(mm3(Q, Qi), f);
-            v3<double> Qim = mv(Qi, mo);
-            v3<double> mip = mv(Xi, Qim);
-            m3<double> K12 = mscl(-1.0, mm3(skew3(fip), Xi));
-            m3<double> dy;
-#pragma unroll
-            for (int i = 0; i < 9; i++) dy.a[i] = 0.0;
-            add_outer(dy, 1.0, Qim, alpha);
-            m3<double> K22 = mscl(-0.5 * g, madd(skew3(Qim), mm3(Xi, dy)));
-            const double q6[6] = {fip.x, fip.y, fip.z, mip.x, mip.y, mip.z};
-            vec_add_n<6>(r, R, q6);
-            int R18[18], C18[18];
-            double V18[18];
-#pragma unroll
-            for (int i = 0; i < 3; i++)
-#pragma unroll
-                for (int j = 0; j < 3; j++) {
-                    R18[3 * i + j] = R[i];
-                    C18[3 * i + j] = R[3 + j];
-                    V18[3 * i + j] = -K12.a[3 * i + j];
-                    R18[9 + 3 * i + j] = R[3 + i];
-                    C18[9 + 3 * i + j] = R[3 + j];
-                    V18[9 + 3 * i + j] = -K22.a[3 * i + j];
-                }
-            gm_add_n<18>(gm, R18, C18, V18);
-        }
+    for (int i = 0; i < 6; i++) {
+        R[i] = dof[6 * L.node[k] + i];
+        q6[i] = q[i];
     }
+    vec_add_n<6>(r, R, q6);
+#pragma unroll
+    for (int i = 0; i < 18; i++) {
+        R18[i] = R[i / 3];
+        C18[i] = R[3 + i % 3];
+        V18[i] = q[6 + i];
+    }
+    gm_add_n<18>(gm, R18, C18, V18);
 }
 
 // Max-norms of a vector over band rows split by DOF kind (translation /
@@ -192,13 +133,37 @@ template <int NV> __device__ __forceinline__ void block_amax(double (&v)[NV], un
 // each Newton iteration (3.9 and 1.6 us).  Only atomics pass between the
 // workgroups, so no fence: one here writes an XCD's whole L2 back (8 us after a
 // 10,000-element assembly).
-__global__ __launch_bounds__(256) void scan_kernel(int n, const double *__restrict__ v, const int *__restrict__ row_nc,
-                                                   unsigned long long *scal, unsigned long long *host)
+//
+// LOADS: the nodal loads, formed beside the first beam launch (ln_out), are added here,
+// row by row: row i takes entry row_load[i] (6 k + component, or -1) and its three
+// tangent entries, where they are not zero.  (As a launch of their own the loads are a
+// chain of six dependent reads: 7.4 us at 777 loaded elements, 10.4 at 10,000; so they
+// cost the scan 0.1 and 2.4 us and the beam launch 0.1 and 1.)
+template <bool LOADS>
+__global__ __launch_bounds__(256) void scan_kernel(int n, double *__restrict__ v, const int *__restrict__ row_nc,
+                                                   unsigned long long *scal, unsigned long long *host,
+                                                   const int *__restrict__ row_load, const double *__restrict__ ln_out,
+                                                   const int *__restrict__ dof, gf_gmat gm)
 {
     unsigned long long *out = scal + GF_SCAL_RES;
     double m[3] = {0.0, 0.0, 0.0};  // translations, rotations, non-finite
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        double a = fabs(v[i]);
+        double a = v[i];
+        if (LOADS) {
+            const int li = row_load[i];
+            if (li >= 0) {
+                const int k = li / 6, c = li - 6 * k, node = row_nc[i] / 6;
+                const double *o = ln_out + (size_t)GF_NODAL_OUT * k;
+                a += o[c];
+                v[i] = a;
+                const double K3[3] = {o[6 + 3 * c], o[7 + 3 * c], o[8 + 3 * c]};
+                if (K3[0] != 0.0 || K3[1] != 0.0 || K3[2] != 0.0) {
+                    const int R3[3] = {i, i, i}, C3[3] = {dof[6 * node + 3], dof[6 * node + 4], dof[6 * node + 5]};
+                    gm_add_n<3>(gm, R3, C3, K3);
+                }
+            }
+        }
+        a = fabs(a);
         if (!(a == a) || a >= 1e300) m[2] = 1.0;
         else if (row_nc[i] % 6 < 3) m[0] = fmax(m[0], a);
         else m[1] = fmax(m[1], a);
@@ -357,8 +322,7 @@ int gf_nodal_loads(gf_model *m, const double *tp)
 {
     if (m->n_load_nodes == 0) return GF_OK;
     hipLaunchKernelGGL(nodal_loads_kernel, dim3((m->n_load_nodes + 127) / 128), dim3(128), 0, m->stream,
-                       m->n_load_nodes, m->d_ln_node, m->d_ln_off, m->d_ln_ids, m->d_lrec, m->d_tab_t, m->d_tab_v,
-                       m->d_disp, m->d_copy, m->d_dof, gf_model_gmat(m), m->d_r, tp);
+                       gf_nodal_of(m, tp), m->d_dof, gf_model_gmat(m), m->d_r);
     GF_HIP(hipGetLastError());
     return GF_OK;
 }
@@ -368,8 +332,10 @@ int gf_nodal_loads(gf_model *m, const double *tp)
 // are zero afterwards.
 int gf_scan_residual(gf_model *m)
 {
-    hipLaunchKernelGGL(scan_kernel, dim3(grid_for(m->n_free, 256, 128)), dim3(256), 0, m->stream, m->n_free, m->d_r,
-                       m->d_row_nc, (unsigned long long *)m->d_scal, (unsigned long long *)m->h_scal);
+    hipLaunchKernelGGL(m->d_ln_out ? scan_kernel<true> : scan_kernel<false>, dim3(grid_for(m->n_free, 256, 128)),
+                       dim3(256), 0, m->stream, m->n_free, m->d_r, m->d_row_nc, (unsigned long long *)m->d_scal,
+                       (unsigned long long *)m->h_scal, (const int *)m->d_row_load, (const double *)m->d_ln_out,
+                       (const int *)m->d_dof, gf_model_gmat(m));
     GF_HIP(hipGetLastError());
     return GF_OK;
 }
