@@ -126,8 +126,9 @@ __global__ __launch_bounds__(SPLIT ? 2 * WG : WG) void beam_assemble_kernel(
     const bool pair = w0 && tid < 9 * EPB && e2 < e1;
     double w = 0.0, Na2[2], Nb2[2], dNa2[2], dNb2[2];
     m3<double> T2;
-    double old36[36], *base36 = gm.layout == GM_BTD ? gm.A : gm.ab;
-    unsigned off36[36];  // entries from base36 (both layouts hold fewer than 2^32)
+    double old36[36], *base36 = gm_base(gm);
+    size_t row6[6];  // entry (i, j) of the pair: base36[row6[i] + step36[6 i + j]]
+    unsigned step36[36];
     bool okr[6], okc[6];
     auto fetch = [&] {
         if (!pair) return;
@@ -151,19 +152,9 @@ __global__ __launch_bounds__(SPLIT ? 2 * WG : WG) void beam_assemble_kernel(
                 okr[k] = rr[k] >= 0;
                 okc[k] = cc[k] >= 0;
             }
-            int R36[36], C36[36];
+            gm_pair(gm, rr, cc, row6, step36);
 #pragma unroll
-            for (int k = 0; k < 36; k++) {
-                R36[k] = rr[k / 6];
-                C36[k] = cc[k % 6];
-            }
-            double *p36[36];
-            gm_addr_n<36>(gm, R36, C36, p36);
-#pragma unroll
-            for (int k = 0; k < 36; k++) {
-                off36[k] = (unsigned)(p36[k] - base36);
-                old36[k] = base36[off36[k]];
-            }
+            for (int k = 0; k < 36; k++) old36[k] = base36[row6[k / 6] + step36[k]];
         }
     };
     if (SPLIT) fetch();
@@ -290,7 +281,7 @@ __global__ __launch_bounds__(SPLIT ? 2 * WG : WG) void beam_assemble_kernel(
 #pragma unroll
                 for (int j = 0; j < 6; j++)
                     if (okr[i] && okc[j])
-                        base36[off36[6 * i + j]] = old36[6 * i + j] + blk[2 * (i / 3) + j / 3].a[3 * (i % 3) + j % 3];
+                        base36[row6[i] + step36[6 * i + j]] = old36[6 * i + j] + blk[2 * (i / 3) + j / 3].a[3 * (i % 3) + j % 3];
         } else {
             double *Ke = Kout + (size_t)e2 * 324;
 #pragma unroll

@@ -8,6 +8,7 @@
 #include <thread>
 #include <vector>
 #include "../../include/giraffe_amd.h"
+#include "gf_index.h"
 
 // Mixed precision: FP64 factorisations in a row after two FP32 fallbacks in a
 // row (the first back-off; later ones double while the retries keep failing).
@@ -84,24 +85,7 @@ enum {
 // Gauss-point state of Beam_1, [BG_COUNT][nb]: per gp Q_i(9) kappa_i(3) z'_i(3)
 enum { BG_PER_GP = 15, BG_COUNT = 30 };
 
-// ---- global tangent storage -------------------------------------------------
-// GM_BTD : block-tridiagonal blocks A (sub), B (diag), C (super), [nblk][m][m]
-//          row-major, consecutive in one allocation (B = A + nblk m m,
-//          C = B + nblk m m); used when the half-bandwidth fits a block of m <= 32.
-// GM_BAND: skewed dense band, entry (i, c) with -hb <= c - i <= ku at
-//          ab[i * ld + c + hb], ld = hb + ku (each row a contiguous window of
-//          ld + 1); ku = gf_band_ku(hb) leaves room for the factorisation's
-//          fill.  Sub-matrices inside the band are plain strided matrices with
-//          leading dimension ld, which is what the band LU tiles use.
-enum { GM_BTD = 0, GM_BAND = 1 };
-struct gf_gmat {
-    int layout;
-    int m;
-    double *A, *B, *C;
-    double *ab;
-    int hb;
-    int ld;
-};
+// ---- global tangent storage (gf_index.h) --------------------------------------
 int gf_band_ku(int hb);
 
 // Reciprocal of a pivot that is finite, non-zero and not subnormal (the solvers
@@ -121,49 +105,6 @@ __device__ __forceinline__ float pivot_rcp(float p)
     float r = __builtin_amdgcn_rcpf(p);
     const float e = fmaf(-p, r, 1.0f);
     return fmaf(r, e, r);
-}
-
-// Block index q = floor(x / m) for 0 <= x < 2^24 and m <= 32, through a float
-// product (one rounding, then one correction step each way): no integer divide.
-__device__ __forceinline__ int gm_block_of(int x, int m, float inv_m)
-{
-    int q = (int)(((float)x + 0.5f) * inv_m);
-    q -= q * m > x ? 1 : 0;
-    q += (q + 1) * m <= x ? 1 : 0;
-    return q;
-}
-
-// Addresses of N entries (R, Cc); a constrained entry (R or Cc negative) gets a
-// valid stand-in address whose value is never stored back.  The layout test is
-// one uniform branch around the whole batch, so loads through the addresses are
-// straight-line code and all in flight together.
-template <int N>
-__device__ __forceinline__ void gm_addr_n(const gf_gmat &g, const int (&R)[N], const int (&Cc)[N], double *(&p)[N])
-{
-    if (g.layout == GM_BTD) {
-        const int m = g.m;
-        const float inv_m = 1.0f / (float)m;
-        const ptrdiff_t stride = g.B - g.A;
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-            const bool ok = R[k] >= 0 && Cc[k] >= 0;
-            const int r = ok ? R[k] : 0, c = ok ? Cc[k] : 0;
-            const int bi = gm_block_of(r, m, inv_m), bj = gm_block_of(c, m, inv_m);
-            const size_t off = ((size_t)bi * m + (r - bi * m)) * m + (c - bj * m);
-            // A, B and C are one allocation in that order (gf_btd_alloc): the block
-            // kind selects an offset; a selected pointer would be re-read from the
-            // kernel arguments, one dependent load per entry
-            const ptrdiff_t kind = bj < bi ? 0 : (bj == bi ? 1 : 2);
-            p[k] = g.A + kind * stride + off;
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-            const bool ok = R[k] >= 0 && Cc[k] >= 0;
-            const int r = ok ? R[k] : 0, c = ok ? Cc[k] : 0;
-            p[k] = g.ab + (size_t)r * (size_t)g.ld + (size_t)(c + g.hb);
-        }
-    }
 }
 
 // N entries added at once: every address, all loads, then the stores of the
