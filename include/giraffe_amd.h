@@ -346,7 +346,13 @@ int gf_bandsystem(int n, int hb, const double *ab_rows, const double *b, double 
  * models use (no counterpart in the reference; a test entry point): nblk block
  * rows of m x m row-major blocks, A[i] coupling row i to i-1 (A[0] ignored),
  * B[i] the diagonal, C[i] coupling to i+1 (C[nblk-1] ignored), 1 <= m <= 32.
- * info_fail = 1 on a zero or non-finite pivot. */
+ * info_fail = 1 on a zero or non-finite pivot.
+ * Accuracy: a reduced diagonal block is eliminated with its diagonal pivots while
+ * no multiplier exceeds 16 and no pivot its row's diagonal entry more than twice,
+ * else with row interchanges within the block wherever a pivot is below half of its
+ * column's largest entry.  Blocks are not exchanged with their neighbours: a reduced
+ * diagonal block that is singular, or nearly so, in a regular system costs digits as
+ * its condition does (a zero pivot: info_fail). */
 int gf_btdsystem(int m, int nblk, const double *A, const double *B, const double *C, const double *b, double *x,
                  int *info_fail);
 /* gf_btdsystem on the caller's DEVICE buffers, allocating nothing.  No
