@@ -174,7 +174,7 @@ __device__ __forceinline__ void cr_pivot(double (&r)[H][NC], double (&sc)[H], in
 // rows with -8 below the diagonal and ones in the last column lose every digit
 // in 16 pivots); with both limits the entries of a column are at most 32 times its
 // original diagonal entry when it is eliminated, however rows and columns are
-// scaled.  Errors against long double of 150,000 random, sparse, graded and symmetric
+// scaled.  Errors against long double of 100,000 random, sparse, graded and symmetric
 // blocks of 3 to 32 rows, in ulp times the condition: the 99th percentile of
 // those that pass both limits is 1.4 to 3.3 by family, with interchanges for the
 // same blocks 1.9 to 13; and no row of risers and roll-ups fails the second limit.

@@ -291,7 +291,8 @@ __device__ __forceinline__ int live_rows(const gf_front_dev &F, int p) { return 
 
 // A child's Schur complement entries of a tile at a thread's result positions:
 // first the positions in the child's update rows, then, behind a product, the
-// entries.
+// entries (at 64-bit addresses: a front may pass 4 GB, and 32-bit offsets were no
+// faster, 153.2 ms a 64 x 64 plate solve against 152.9).
 template <typename T> struct ChildTile {
     int a[2][4], b[2];
     __device__ __forceinline__ void positions(const FrontTab &t, int c, int R0, int C0)
@@ -308,11 +309,11 @@ template <typename T> struct ChildTile {
     __device__ __forceinline__ void entries(const FrontTab &t, int c, const T *Fb, T (&u)[2][2][4])
     {
         const gf_front_dev C = t.fr[t.child[c]];
-        const T *U = Fb + C.F + (size_t)(NB * C.kb) * C.mp + NB * C.kb;
+        const T *U = Fb + C.F + gf_front_at(NB * C.kb, NB * C.kb, C.mp);
         acc_each<T>([&](int x, int y, int v, int, int) {
             u[x][y][v] = T(0);
             if (a[x][v] >= 0 && b[y] >= 0)
-                u[x][y][v] = at(U, ((unsigned)a[x][v] * (unsigned)C.mp + (unsigned)b[y]) * (unsigned)sizeof(T));
+                u[x][y][v] = U[gf_front_at(a[x][v], b[y], C.mp)];
         });
     }
 };
@@ -359,7 +360,7 @@ __global__ __launch_bounds__(256, 3) void front_step_kernel(FrontTab t, int firs
     // product 1: W = E_q A'(q, j), q = p (update, diagonal) or p - 1 (conversion)
     const int q = kind == 2 ? ti : p, ka = live_rows(F, q);
     const T *E = Ef + (size_t)q * NB * NB;
-    const T *Aq = A + (size_t)(q * NB * ld) + C0;  // A'(q, j)
+    const T *Aq = A + gf_front_at(q * NB, C0, F.mp);  // A'(q, j)
     T e[16], a0[8], a1[8];
 #pragma unroll
     for (int r = 0; r < 16; r++) e[r] = at(E + 256 * r, tid * (unsigned)sizeof(T));
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(256, 3) void front_step_kernel(FrontTab t, int firs
     rowchunk_put_t(sm.C, a0);
     __syncthreads();
     T l0[8], l1[8], old[2][2][4];
-    const T *Lp = A + (size_t)(ti * NB * ld) + p * NB;  // L(i, p)
+    const T *Lp = A + gf_front_at(ti * NB, p * NB, F.mp);  // L(i, p)
     colchunk_load(l0, Lp, ld, 0);  // (a conversion item does not use it)
     if (rhs_row && tid < NB) {
         double yv = 0.0;
@@ -378,7 +379,7 @@ __global__ __launch_bounds__(256, 3) void front_step_kernel(FrontTab t, int firs
         if (kind == 2) Vb[F.V + (size_t)(q * NB) + tid] = yv;
         else rv[1][tid] = yv;  // y_p
     }
-    auto tile = [&](int i0) { return A + (size_t)(i0 * NB * ld) + C0; };
+    auto tile = [&](int i0) { return A + gf_front_at(i0 * NB, C0, F.mp); };
     Acc<T> w;
     w.zero();
     mm_xc<T>(w, sm.X, sm.C, 0, ka);

@@ -104,3 +104,8 @@ GF_HD void gm_pair(const gf_gmat &g, const int (&R)[6], const int (&C)[6], size_
         }
     }
 }
+
+// Entry (i, j) of a front with rows of mp entries: 64 bits, as fronts of more than
+// 23,170 rows pass 4 GB (forced multifrontal plans of meshes whose coordinates do not
+// separate them) and of more than 65,535 rows 2^32 entries.
+GF_HD size_t gf_front_at(int i, int j, int mp) { return (size_t)i * (size_t)mp + (size_t)j; }

@@ -80,3 +80,26 @@ def test_block_rows(pair, m, nf):
             kind = 1 + (c // m > r // m) - (c // m < r // m)
             if abs(c // m - r // m) <= 1:
                 assert got[k] == kind * npad * m + r * m + c % m
+
+
+_FRONT = r'''
+#include <cstdio>
+#include "gf_index.h"
+int main()
+{
+    int i, j, mp;
+    while (scanf("%d %d %d", &i, &j, &mp) == 3) printf("%llu\n", (unsigned long long)(8 * gf_front_at(i, j, mp)));
+}
+'''
+
+
+def test_front_entries(tmp_path):
+    """Byte offsets of FP64 entries around 2^32 bytes (23,170 rows) and 2^32 entries."""
+    src, exe = tmp_path / "front.cpp", tmp_path / "front"
+    src.write_text(_FRONT)
+    subprocess.check_call(["g++", "-std=c++17", "-Wno-unknown-pragmas", "-I", CSRC, str(src), "-o", str(exe)])
+    cases = [(i, j, mp) for mp in (64, 23168, 23232, 25472, 65472, 65536, 70016) for i in (0, 63, mp // 2, mp - 1)
+             for j in (0, mp - 1)]
+    out = subprocess.run([str(exe)], input="\n".join("%d %d %d" % c for c in cases), capture_output=True, text=True,
+                         check=True).stdout
+    assert [int(v) for v in out.split()] == [8 * (i * mp + j) for i, j, mp in cases]
