@@ -53,7 +53,7 @@ struct CrArgs {
 
 typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
-template <int H, int R> struct CrSmem {
+template <int H, int R> struct alignas(16) CrSmem {
     static constexpr int MT = 16 * H, LD = MT + 2, SLOTS = crc<H, R>::SLOTS;
     // strides of 2 mod 16 doubles: sixteen lanes reading 16 bytes of sixteen rows hit distinct banks
     double A[SLOTS][MT * LD], B[SLOTS][MT * LD], C[SLOTS][MT * LD];

@@ -67,7 +67,7 @@ __device__ __forceinline__ double child_sum(const FrontTab &t, const gf_front_de
 
 // LDS of the assembly kernel: the first diagonal block of a front and the
 // inverse's scratch.
-template <typename T> struct AsmSmem {
+template <typename T> struct alignas(16) AsmSmem {
     T P[NB * LDT];
     T tmp[INV_TMP];
     T aux[4 + NB];
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(ASM_T, 6) void front_assemble_kernel(FrontTab t, in
 // for which the MFMA operand reads (16 rows x 4 consecutive entries) hit distinct
 // banks; a B operand is kept transposed so that it is read the same way.  The
 // inverse's scratch reuses C.
-template <typename T> struct FStepSmem {
+template <typename T> struct alignas(16) FStepSmem {
     T X[NB * LDT];
     union {
         T C[NB * SA_LD];
@@ -585,7 +585,8 @@ template <typename T> struct RowTile {
             v[2 * k + 1] = w.y;
         }
     }
-    // acc[k] += this lane's part of row 2 k + l / 32 times y (LDS, the tile's 64 columns)
+    // acc[k] += this lane's part of row 2 k + l / 32 times y (LDS, 16-byte aligned; the tile's
+    // 64 columns)
     __device__ __forceinline__ void dot(double (&acc)[8], const double *y) const
     {
         const double2 w = *reinterpret_cast<const double2 *>(y + 2 * (threadIdx.x & 31));
@@ -621,7 +622,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void front_bwd_upd_kernel(FrontTab t, int first, const T *Fb, const T *Eb,
                                                             const double *x, double *Vb, int raw_last)
 {
-    __shared__ double xu[KMAX];
+    __shared__ alignas(16) double xu[KMAX];
     const int *it = t.items + 4 * (size_t)(first + blockIdx.x);
     const gf_front_dev F = t.fr[it[0]];
     const int p = it[1], tid = threadIdx.x, r = tile_row();
@@ -672,7 +673,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void front_bwd_own_kernel(FrontTab t, int f0, const T *Fb, const T *Eb,
                                                             const double *Vb, double *x, int raw_last)
 {
-    __shared__ double y[KMAX];
+    __shared__ alignas(16) double y[KMAX];
     const int f = f0 + blockIdx.x;
     const gf_front_dev F = t.fr[f];
     const int kp = NB * F.kb, tid = threadIdx.x, r = tile_row();

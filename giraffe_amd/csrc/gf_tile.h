@@ -310,7 +310,7 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_wave_barrier();
 }
 
-// In-place inverse of the 64 x 64 matrix M ([64][LDT]) by 256 threads: block
+// In-place inverse of the 64 x 64 matrix M ([64][LDT], 16-byte aligned) by 256 threads: block
 // Gauss-Jordan over 16 x 16 blocks.  Step kb, with the pivot block P already
 // inverted in place and the column blocks C_i = M(i, kb) (i != kb) saved: row
 // blocks R_j = P^-1 M(kb, j), M(i, j) -= C_i R_j, M(i, kb) = -C_i P^-1 (MFMA
@@ -487,7 +487,7 @@ template <typename T> __device__ __forceinline__ void tile_put(T *dst, int ld, c
 // block D for the inverse), Q B operands (A'(p, j), then U(p, j)); the
 // inverse's scratch reuses Q.  75 KB in FP64, so two workgroups share a CU and
 // a launch's tiles are all resident at once.
-template <typename T> struct StepSmem {
+template <typename T> struct alignas(16) StepSmem {
     T P[NB * LDT];
     union {
         T Q[NB * LDQ];
