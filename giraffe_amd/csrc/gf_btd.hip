@@ -597,13 +597,17 @@ static int btd_factor_t(gf_btd &b, hipStream_t s, int *d_flag)
     int launches = 0;
     for (int L = 0; L < b.tail_level; L++) {
         const int nL = b.lvl_n[L];
+        const int pr = gf_probe_begin(s, GF_KC_BTD_LEVEL);
         hipLaunchKernelGGL((btd_level_kernel<T, MT>), dim3(nL / 2), dim3(128), 0, s, F, L, nL, Lsv + b.lvl_save[L] * bs,
                            Rsv + b.lvl_save[L] * bs);
+        gf_probe_end(s, pr, nL / 2);
         launches++;
     }
     const int nL0 = b.tail_level < b.levels ? b.lvl_n[b.tail_level] : 1;
+    const int pr = gf_probe_begin(s, GF_KC_BTD_TAIL);
     hipLaunchKernelGGL((btd_tail_kernel<T, MT>), dim3(1), dim3(128 * cfg<MT>::PAIRS), 0, s, F, b.tail_level, b.levels,
                        nL0, Lsv, Rsv, (const long long *)b.d_save);
+    gf_probe_end(s, pr, nL0);
     GF_HIP(hipGetLastError());
     return launches + 1;
 }

@@ -271,8 +271,10 @@ int gf_timing_read(gf_model *m, double *ms_out, long long *launches_out, int res
  * accumulated milliseconds, launches, and work units (GF_KC_* comments). */
 #define GF_KC_BTD_LEVEL      0  /* cr_reduce_kernel<, , false>; unit: block row eliminated,
                                    counted in halvings of the rows down to 16 (a launch
-                                   runs three to five)                              */
-#define GF_KC_BTD_TAIL       1  /* cr_reduce_kernel<, , true>; unit: block row eliminated */
+                                   runs three to five).  Mixed precision: also the FP32
+                                   factorisation's btd_level_kernel, a halving each  */
+#define GF_KC_BTD_TAIL       1  /* cr_reduce_kernel<, , true>, btd_tail_kernel; unit: block
+                                   row eliminated                                   */
 #define GF_KC_BAND_PANEL     2  /* band_batch_inv_kernel; unit: flop of the batch inverses */
 #define GF_KC_BAND_UPDATE    3  /* band_step_kernel; unit: band column eliminated   */
 #define GF_KC_BAND_SWEEP     4  /* band_batch_apply_kernel, band_couple_kernel; unit: row
@@ -284,7 +286,7 @@ int gf_timing_read(gf_model *m, double *ms_out, long long *launches_out, int res
                                    factorisations, sum over eliminated columns c of
                                    2 (m - c - 1)^2 for a front of order m            */
 #define GF_KC_FRONT_ASSEMBLE 8  /* front_assemble_kernel; unit: front entry written */
-#define GF_KC_FRONT_SOLVE    9  /* front_fwd_own/fwd_upd/bwd_upd/bwd_own_kernel; unit: factor
+#define GF_KC_FRONT_SOLVE    9  /* front_fwd_own/fwd_upd/bwd_upd/bwd_own/bwd_kernel; unit: factor
                                    byte read (own triangle with the diagonal inverses,
                                    or the update panel)                              */
 #define GF_NKC              10
