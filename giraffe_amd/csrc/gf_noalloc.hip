@@ -20,7 +20,7 @@ namespace {
 // Capacity: nblk * m * m <= 2^17 block entries (so n = nblk m <= 2^17 rows).
 constexpr size_t NA_ELEMS = (size_t)1 << 17;
 // X|Y of every row (2 E), then the reduced rows of each level (at most a quarter
-// of the rows before): under 2.92 E over all sizes within the capacity.  Then a
+// of the rows before): under 2.93 E over all sizes within the capacity.  Then a
 // stand-in for a solution or flag that overlaps the inputs (at most E, and a
 // line): 4.2 MB in all.
 constexpr size_t NA_WORK = 3 * NA_ELEMS, NA_SCRATCH = 4 * NA_ELEMS + 32;
@@ -61,6 +61,10 @@ extern "C" int gf_btdsystem_noalloc(int m, int nblk, const double *A, const doub
                                     const double *b, double *x, int *info_fail, void *stream)
 {
     if (m < 1 || m > 32 || nblk < 1 || !A || !B || !C || !b || !x || !info_fail) return GF_E_ARG;
+    if (b == x) {  // (before anything is enqueued: the flag of a refused call is not written)
+        gf_set_error("gf_btdsystem_noalloc: x must differ from b");
+        return GF_E_ARG;
+    }
     if ((size_t)nblk * m * m > NA_ELEMS) {
         gf_set_error("gf_btdsystem_noalloc: nblk * m * m exceeds the scratch capacity of 131072");
         return GF_E_CAPACITY;
@@ -88,7 +92,7 @@ extern "C" int gf_btdsystem_noalloc(int m, int nblk, const double *A, const doub
     auto meets = [&](const void *p, size_t np) {
         return overlap(p, np, A, E) || overlap(p, np, B, E) || overlap(p, np, C, E) || overlap(p, np, b, n);
     };
-    double *xs = meets(x, n) && b != x ? sp + NA_WORK : x;
+    double *xs = meets(x, n) ? sp + NA_WORK : x;
     int *flag = meets(info_fail, 4) ? (int *)(sp + NA_WORK + NA_ELEMS) : info_fail;
     GF_TRY(gf_launch_fill_bytes(s, flag, 4));
     const int l = gf_btd_factor_solve(t, s, flag, b, xs);
