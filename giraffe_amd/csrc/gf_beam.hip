@@ -19,9 +19,10 @@
 // The kernel takes a whole SIMD's registers a wavefront.  While a launch's
 // workgroups all fit the device with two of them (512), a second wavefront runs
 // phases 1 and 3 beside the first's phase 2, whose data, old matrix entries
-// included, is read during phase 1: such a launch is one chain of latencies,
-// 14.2 us with the three phases in a row and 11.7 us so.  Beyond, one wavefront
-// takes the phases in a row (715 workgroups: 23 us, two wavefronts each 27).
+// included, is read during phase 1: such a launch is one chain of latencies
+// (a colour of 777 elements, 56 workgroups: 12.1 us with the three phases in a
+// row, 10.5 us so; 500 workgroups: 18.2 and 17.9).  Beyond, one wavefront takes the
+// phases in a row (715 workgroups: 21.9 us, two wavefronts each 26.4).
 // Elements are sorted by colour (no two elements of a colour share a node),
 // so one launch per colour scatters without atomics and deterministically.
 #include "gf_internal.h"

@@ -362,10 +362,10 @@ int gf_btdsystem(int m, int nblk, const double *A, const double *B, const double
  * memory (code under HIP graph capture, tight serving loops).  A, B, C, b, x
  * and info_fail are device pointers (info_fail: one int, written 0 or 1); the
  * work is enqueued on `stream` (a hipStream_t, NULL for the null stream) and
- * the call returns without waiting.  The factor workspace lives in a fixed
- * device array of the library (4.2 MB on each GPU it runs on, held until the
- * process ends): nblk * m * m <= 131072, else GF_E_CAPACITY before any device
- * work.  Calls that overlap on one GPU share that array and race. */
+ * the call returns without waiting.  x must not be b (GF_E_ARG); it may overlap
+ * the inputs otherwise.  The workspace lives in a fixed device array of the
+ * library (4.2 MB on each GPU it runs on, held until the process ends):
+ * nblk * m * m <= 131072, else GF_E_CAPACITY before any device work.  Calls that overlap on one GPU share that array and race. */
 int gf_btdsystem_noalloc(int m, int nblk, const double *A, const double *B, const double *C, const double *b,
                          double *x, int *info_fail, void *stream);
 
