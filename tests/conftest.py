@@ -14,6 +14,18 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "slow: longer CPU runs")
 
 
+@pytest.fixture
+def device_holds():
+    """holds(model, solver): skips where the device's memory is below twice the model's footprint."""
+    def holds(model, **kw):
+        import torch
+        from giraffe_amd import runtime
+        total, need = torch.cuda.get_device_properties(0).total_memory, runtime.footprint(model, **kw)
+        if total < 2 * need:
+            pytest.skip(f"{need / 1e9:.0f} GB model on a device of {total / 1e9:.0f} GB")
+    return holds
+
+
 @pytest.fixture(scope="session")
 def oracle_lib():
     import oracle

@@ -76,13 +76,14 @@ def test_static_matches_oracle(oracle_lib, solver, precision):
 
 
 @pytest.mark.parametrize("nq", [24, 172])
-def test_newton_contracts_in_the_last_rows(nq):
+def test_newton_contracts_in_the_last_rows(nq, device_holds):
     """172 x 172 quads: 618,684 free DOFs and 1.04 x 2^32 band entries, the beams in the
     last rows.  With the whole tangent Newton's increments square their relative size
     from one iteration to the next (the first is 2e-3 off at both sizes, so the fourth
     is far below 1e-9 of it); with the beams' terms at other entries they would fall by a
     constant factor."""
     m, _, _ = _stiffened(nq, nq - 1, imperf=0.0, p_max=2e2)
+    device_holds(m)
     dm = runtime.DeviceModel(m)
     dm.set_window(0.0, 1.0)
     dm.begin_step(0.0, 1.0)

@@ -27,8 +27,9 @@ def scattered_plate(nq, seed=0):
 
 
 @pytest.mark.parametrize("nq", [6, 20, 42])
-def test_newton_contracts(nq):
+def test_newton_contracts(nq, device_holds):
     m = scattered_plate(nq)
+    device_holds(m, solver=abi.GF_SOLVER_FRONTS)
     if nq == 42:
         fr = runtime.front_plan(m)["front"].astype(np.int64)
         kp, mp = fr[:, 1], fr[:, 2]
